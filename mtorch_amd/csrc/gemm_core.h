@@ -117,6 +117,10 @@ struct GemmArgs {
   // ResNet block's time embedding), added after the bias and before the residual
   const void* chan_add;
   int64_t chan_add_ld;
+  // fp16 linears of few rows (linear_skinny.hip): halves per load with which its kernel may take
+  // the problem (0: not), and the K its rows hold where K is that rounded up to a whole chunk
+  int rows_vec;
+  int64_t K_rows;
 };
 
 // v as the unfused op sequence reads it back after storing it in T, for the general epilogue

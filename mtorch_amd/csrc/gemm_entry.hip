@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 
 #include "gemm_core.h"
 
@@ -16,10 +17,10 @@ int launch_conv_f32(int device, const GemmArgs& a, hipStream_t s);
 int launch_linear_f16(int device, const GemmArgs& a, hipStream_t s);
 int launch_geglu_f16(int device, const GemmArgs& a, hipStream_t s);
 int launch_gemm_f16(int device, const GemmArgs& a, int64_t batch, bool b_trans, hipStream_t s);
-// The streamed-kernel launcher for linears (linear_stream.hip) and the launcher for few rows
-// (linear_skinny.hip); -1 where they do not apply.
+// The streamed-kernel launcher for linears (linear_stream.hip); -1 where it does not apply.
 int try_stream_linear(int device, const GemmArgs& a, hipStream_t s);
-int try_skinny_linear(int device, const GemmArgs& a, hipStream_t s);
+// How the kernel for few rows may load a linear's operands (linear_skinny.hip).
+int linear_rows_vec(const GemmArgs& a);
 
 namespace {
 
@@ -104,20 +105,28 @@ int mthip_linear(int device, int dtype, const void* x, int64_t lda, const void* 
     a.gelu_tab = gelu_f16_lookup(device, s);
     if (!a.gelu_tab) return fail(MTHIP_ERR_HIP, "mthip_linear: gelu table setup failed");
   }
-  if (dtype == MTHIP_F16) {
-    const int rc = try_skinny_linear(device, a, s);
-    if (rc >= 0) return rc;
-  }
   const int vec = dtype == MTHIP_F16 ? 8 : 4;
   const int64_t es = dtype == MTHIP_F16 ? 2 : 4;
   // the fp32 kernel reads rows of any length and alignment in place
   const bool vec_ok =
       dtype == MTHIP_F32 || (aligned16(x) && aligned16(w) && lda % vec == 0 && ldw % vec == 0 && K % vec == 0);
+  const int64_t Kp = ceil_div(K, vec) * vec;
+  // Few rows: the launchers of the tile GEMM and the streamed GEMM hand the problem on.  Rows of any
+  // even length are read in place where the tile GEMM would take their padded copies.
+  if (dtype == MTHIP_F16) {
+    a.rows_vec = linear_rows_vec(a);
+    a.K_rows = K;
+    // (not where the padded copies would take the streamed GEMM, or no few-row hand-over exists)
+    if (a.rows_vec == 2) {
+      const char* dtl = std::getenv("MTHIP_GEMM_DTL");
+      if ((Kp % 320 == 0 && (act == MTHIP_ACT_NONE || act == MTHIP_ACT_GELU)) || (dtl && dtl[0] == '0')) a.rows_vec = 0;
+    }
+  }
+  const bool in_place = vec_ok || a.rows_vec == 2;
   void* xp = nullptr;
   void* wp = nullptr;
-  if (!vec_ok) {
+  if (!in_place) {
     // Zero-padded aligned copies of both operands (K rounded up to a whole chunk).
-    const int64_t Kp = ceil_div(K, vec) * vec;
     int rc = pad_operand<uint16_t>(device, s, x, 1, M, K, lda, 0, Kp, &xp);
     if (rc == MTHIP_OK) rc = pad_operand<uint16_t>(device, s, w, 1, N, K, ldw, 0, Kp, &wp);
     if (rc != MTHIP_OK) {
@@ -127,15 +136,15 @@ int mthip_linear(int device, int dtype, const void* x, int64_t lda, const void* 
     a.a = xp;
     a.b = wp;
     a.lda = a.ldb = Kp;
-    a.K = Kp;
   }
+  if (dtype == MTHIP_F16) a.K = Kp;
   a.a_bytes = ((M - 1) * a.lda + a.K) * es;
   a.b_bytes = ((N - 1) * a.ldb + a.K) * es;
   int rc;
   if (a.a_bytes > kMaxBufferBytes || a.b_bytes > kMaxBufferBytes)
     rc = fail(MTHIP_ERR_UNSUPPORTED, "mthip_linear: operands above 2 GiB are not supported");
   else if (dtype == MTHIP_F16) {
-    rc = (act == MTHIP_ACT_NONE || act == MTHIP_ACT_GELU) ? try_stream_linear(device, a, s) : -1;
+    rc = (act == MTHIP_ACT_NONE || act == MTHIP_ACT_GELU) && a.rows_vec != 2 ? try_stream_linear(device, a, s) : -1;
     if (rc < 0) rc = launch_linear_f16(device, a, s);
   } else {
     rc = launch_linear_f32(device, a, s);

@@ -13,6 +13,7 @@
 namespace mthip {
 
 int gemm_cu_count(int device);
+int launch_linear_rows(const GemmArgs& a, int mf, hipStream_t s);
 
 namespace {
 
@@ -120,6 +121,9 @@ int launch_tile(int device, GemmArgs a, int64_t batch, hipStream_t s) {
   }
   a.kt_per_split = ceil_div(nk, ksplit);
   a.ksplit = ceil_div(nk, a.kt_per_split);  // no empty slice
+  if constexpr (DS > 0 && MODE == MODE_NT && EPI == EPI_LINEAR) {
+    if (a.rows_vec) return launch_linear_rows(a, 32, s);  // the same slices and bits
+  }
   a.units = tiles * a.ksplit;
   MTHIP_REQUIRE(a.units < (int64_t(1) << 31) && a.N < (int64_t(1) << 31) && a.M < (int64_t(1) << 31),
                 "gemm: problem too large (tiles, rows or columns beyond 2^31)");

@@ -1,162 +1,179 @@
 // fp16 linear with few rows: y[M, N] = act(x[M, K] . w[N, K]^T + b) (+ residual), M <= 16 -- the
 // timestep MLP and the time projections of an SD UNet (M = 2).
 //
-// Bound by the weights' bytes and, at SD sizes, by one memory round trip: the tile GEMM reads the
-// same weights with 20 64x64 tiles on 256 CUs and a K split whose reduction is a second launch
-// (1280x1280: 9.2 + 4.1 us).  Here a wave owns COLS output columns: its lanes take consecutive
-// chunks of the columns' weight rows (16-byte chunks, or 4-byte ones where the rows are only
-// 4-byte aligned, so no padded copies are made) and of the x rows, all loads of a trip issued
-// together, and multiply them in fp32 (v_fma_mix_f32); a butterfly per row and column leaves the
-// sums in every lane, and lane m finishes row m.
+// Returns the bits of the tile GEMM it stands in for: the launchers of the direct-to-LDS GEMM
+// (gemm_launch.h) and of the streamed GEMM (linear_stream.hip) call it after they have chosen their
+// K slices, and a slice runs that kernel's MFMAs (MF = 32: 32x32x16, MF = 16: 16x16x32) over the
+// same K positions in the same order; the slices are summed and finished as
+// gemm_splitk_reduce_kernel does.  An output's sum does not depend on what the other rows and
+// columns of a fragment hold, so a fragment may hold COLS real columns by M real rows.
+//
+// Bound by one memory round trip and the slice's chain of MFMAs (1280x1280, M = 2: 5.4 us, 3.3 MB of
+// weights): a wave owns COLS columns of one slice, so that a layer of SD's sizes has a wave on
+// most SIMDs, issues the weight loads of ten K tiles before it waits for the first, and the slices
+// meet in LDS instead of in a second launch.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstdlib>
 
 #include "gemm_core.h"
-#include "wave_ops.h"
 
 namespace mthip {
 
-int gemm_cu_count(int device);
-
 namespace {
 
-__device__ __forceinline__ float half_at(uint32_t w, int hi) { return h2f_bits((uint16_t)(hi ? w >> 16 : w & 0xffffu)); }
+// A workgroup is one wave per K slice (at most MAXW) over COLS output columns.  V: halves per load (8,
+// or 2 where rows are only 4-byte aligned); T: 64-deep K tiles whose weight loads are in flight
+// together, XT (a divisor of T): tiles whose x is.
+template <int MF, int COLS, int V, int T, int XT, int MAXW, int ACT>
+__global__ __launch_bounds__(64 * MAXW) void linear_rows_kernel(const GemmArgs args) {
+  constexpr int KI = MF == 32 ? 16 : 32, NM = 64 / KI;  // k per MFMA, MFMAs per tile
+  constexpr int NR = MF == 32 ? COLS / 2 : 4;           // accumulator registers that hold real columns
+  constexpr uint32_t kOOB = 0x80000000u;                // beyond every buffer: reads zeros
+  typedef float Acc __attribute__((ext_vector_type(MF == 32 ? 16 : 4)));
+  __shared__ float part[MAXW][16][COLS + 4];
 
-// MT: rows (M <= MT); V: halves per chunk (8 or 2); U: chunks per lane and trip.
-template <int MT, int COLS, int V, int U, int ACT>
-__global__ __launch_bounds__(256) void linear_skinny_kernel(const GemmArgs args) {
-  constexpr int W = V / 2;  // 32-bit words per chunk
-  const int lane = threadIdx.x & 63;
-  const int M = (int)args.M, N = (int)args.N, nch = (int)args.K / V;
-  const int64_t n0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * COLS;
-  if (n0 >= N) return;
-  const uint16_t* X = reinterpret_cast<const uint16_t*>(args.a);
-  const uint16_t* Wt = reinterpret_cast<const uint16_t*>(args.b);
-  float acc[MT][COLS];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int c = 0; c < COLS; ++c) acc[m][c] = 0.0f;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane % MF, hc = lane / MF;
+  const int M = (int)args.M, K = (int)args.K_rows;
+  const int64_t N = args.N, n0 = (int64_t)blockIdx.x * COLS;
+  const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)args.a, (short)0, (int)(((args.M - 1) * args.lda + K) * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)args.b, (short)0, (int)(((N - 1) * args.ldb + K) * 2), 0x00020000);
+  const uint32_t x_off = lr < M ? (uint32_t)(lr * args.lda + hc * 8) * 2u : kOOB;
+  const uint32_t w_off = lr < COLS && n0 + lr < N ? (uint32_t)((n0 + lr) * args.ldb + hc * 8) * 2u : kOOB;
+  const int kt0 = wave * (int)args.kt_per_split;
+  const int nkt = min((int)args.kt_per_split, (int)ceil_div(args.K, 64) - kt0);
 
-  auto load = [&](const uint16_t* row, int ch, bool ok, uint32_t (&d)[W]) {
-#pragma unroll
-    for (int i = 0; i < W; ++i) d[i] = 0u;
-    if (!ok) return;
+  // The 8 halves at element k of the row at byte offset off (zeros past K).
+  auto load = [&](const __amdgpu_buffer_rsrc_t& r, uint32_t off, int k) -> halfx8 {
+    uint4 u;
     if constexpr (V == 8) {
-      const uint4 u = *reinterpret_cast<const uint4*>(row + (int64_t)ch * V);
-      d[0] = u.x;
-      d[1] = u.y;
-      d[2] = u.z;
-      d[3] = u.w;
+      const uint32_t o = k < K ? off + (uint32_t)(k - hc * 8) * 2u : kOOB;
+      u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off == kOOB ? kOOB : o), 0, 0));
     } else {
-      d[0] = *reinterpret_cast<const uint32_t*>(row + (int64_t)ch * V);
-    }
-  };
-  for (int t0 = 0; t0 < nch; t0 += 64 * U) {
-    uint32_t w[U][COLS][W];
+      uint32_t d[4];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int c = 0; c < COLS; ++c) {
-        const int ch = t0 + u * 64 + lane;
-        const int64_t n = n0 + c < N ? n0 + c : N - 1;
-        load(Wt + n * args.ldb, ch, ch < nch, w[u][c]);
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t o = k + 2 * i < K ? off + (uint32_t)(k - hc * 8 + 2 * i) * 2u : kOOB;
+        d[i] = __builtin_amdgcn_raw_buffer_load_b32(r, (int)(off == kOOB ? kOOB : o), 0, 0);
       }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int ch = t0 + u * 64 + lane;
-      uint32_t x[MT][W];
-#pragma unroll
-      for (int m = 0; m < MT; ++m) load(X + (int64_t)(m < M ? m : M - 1) * args.lda, ch, ch < nch, x[m]);
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int c = 0; c < COLS; ++c)
-#pragma unroll
-          for (int i = 0; i < W; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) acc[m][c] = fmaf(half_at(x[m][i], h), half_at(w[u][c][i], h), acc[m][c]);
+      u = make_uint4(d[0], d[1], d[2], d[3]);
     }
-  }
-  float mine[COLS];  // row `lane`'s sums
-#pragma unroll
-  for (int c = 0; c < COLS; ++c) {
-    mine[c] = 0.0f;
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const float v = wave_sum(acc[m][c]);
-      mine[c] = lane == m ? v : mine[c];
-    }
-  }
-  if (lane >= M) return;
+    return __builtin_bit_cast(halfx8, u);
+  };
+
+  // a thread's outputs below lie in one column: its bias arrives under the products
   const uint16_t* bias = reinterpret_cast<const uint16_t*>(args.bias);
+  const int64_t n = n0 + threadIdx.x % COLS;
+  const uint16_t bias_h = bias && n < N ? bias[n] : 0x8000u;  // (-0 leaves every value as it is)
+
+  Acc acc;
+#pragma unroll
+  for (int r = 0; r < (MF == 32 ? 16 : 4); ++r) acc[r] = 0.0f;
+  for (int t0 = 0; t0 < nkt; t0 += T) {
+    halfx8 w[T][NM];
+    auto tile_k = [&](int t, int kk) {  // (K: zeros)
+      return t0 + t < nkt ? (kt0 + t0 + t) * 64 + kk * KI + hc * 8 : K;
+    };
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int kk = 0; kk < NM; ++kk) w[t][kk] = load(w_rsrc, w_off, tile_k(t, kk));
+    __builtin_amdgcn_sched_barrier(0);  // every load of the trip in flight before the first is waited for
+#pragma unroll
+    for (int h = 0; h < T; h += XT) {
+      halfx8 x[XT][NM];
+#pragma unroll
+      for (int t = 0; t < XT; ++t)
+#pragma unroll
+        for (int kk = 0; kk < NM; ++kk) x[t][kk] = load(x_rsrc, x_off, tile_k(h + t, kk));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < XT; ++t) {
+        if (t0 + h + t >= nkt) break;
+#pragma unroll
+        for (int kk = 0; kk < NM; ++kk) {
+          if constexpr (MF == 32)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[h + t][kk], x[t][kk], acc, 0, 0, 0);
+          else
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[h + t][kk], x[t][kk], acc, 0, 0, 0);
+        }
+      }
+    }
+  }
+  // lane's accumulator: row lr, columns 8 (r / 4) + 4 hc + r % 4 (MF = 16: 4 hc + r)
+  if (lr < M) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) part[wave][lr][8 * (r >> 2) + 4 * hc + (r & 3)] = acc[r];
+  }
+  __syncthreads();
+  if (n >= N) return;
   const uint16_t* res = reinterpret_cast<const uint16_t*>(args.residual);
   uint16_t* Y = reinterpret_cast<uint16_t*>(args.c);
-#pragma unroll
-  for (int c = 0; c < COLS; ++c) {
-    const int64_t n = n0 + c;
-    if (n >= N) continue;
+  const int c = threadIdx.x % COLS;
+  const float b = h2f_bits(bias_h);
+  for (int m = threadIdx.x / COLS; m < M; m += blockDim.x / COLS) {
+    float v = part[0][m][c];
+    for (int k = 1; k < (int)args.ksplit; ++k) v += part[k][m][c];
     NarrowExact narrow;
-    const float b = bias ? h2f_bits(bias[n]) : -0.0f;
-    const uint32_t h = res ? epi_chain_h<EPI_LINEAR, ACT, false, true>(mine[c], b, 0.0f, h2f_bits(res[lane * args.ld_res + n]),
+    const uint32_t h = res ? epi_chain_h<EPI_LINEAR, ACT, false, true>(v, b, 0.0f, h2f_bits(res[m * args.ld_res + n]),
                                                                       args.gelu_tab, narrow)
-                           : epi_chain_h<EPI_LINEAR, ACT, false, false>(mine[c], b, 0.0f, 0.0f, args.gelu_tab, narrow);
-    Y[lane * args.ldc + n] = (uint16_t)h;
+                           : epi_chain_h<EPI_LINEAR, ACT, false, false>(v, b, 0.0f, 0.0f, args.gelu_tab, narrow);
+    Y[m * args.ldc + n] = (uint16_t)h;
   }
 }
 
-template <int MT, int V, int ACT>
-int launch(const GemmArgs& a, int cus, hipStream_t s) {
-  // two columns a wave (each x chunk read once for both) where one column a wave would still
-  // leave every SIMD four waves
-  constexpr int U = V == 8 ? (MT <= 4 ? 3 : 1) : 4;
-  if (a.N >= (int64_t)cus * 32) {
-    hipLaunchKernelGGL((linear_skinny_kernel<MT, 2, V, U, ACT>), dim3((unsigned)ceil_div(a.N, 8)), dim3(256), 0, s, a);
-  } else {
-    hipLaunchKernelGGL((linear_skinny_kernel<MT, 1, V, U, ACT>), dim3((unsigned)ceil_div(a.N, 4)), dim3(256), 0, s, a);
-  }
-  return check_launch("linear_skinny_kernel");
-}
-
-template <int MT, int V>
-int launch_act(const GemmArgs& a, int cus, hipStream_t s) {
+template <int MF, int COLS, int V, int T, int XT, int MAXW>
+int launch(const GemmArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)ceil_div(a.N, COLS)), block((unsigned)(64 * a.ksplit));
   switch (a.act) {
-    case MTHIP_ACT_GELU: return launch<MT, V, MTHIP_ACT_GELU>(a, cus, s);
-    case MTHIP_ACT_GELU_TANH: return launch<MT, V, MTHIP_ACT_GELU_TANH>(a, cus, s);
-    case MTHIP_ACT_SILU: return launch<MT, V, MTHIP_ACT_SILU>(a, cus, s);
-    default: return launch<MT, V, MTHIP_ACT_NONE>(a, cus, s);
+    case MTHIP_ACT_GELU:
+      hipLaunchKernelGGL((linear_rows_kernel<MF, COLS, V, T, XT, MAXW, MTHIP_ACT_GELU>), grid, block, 0, s, a);
+      break;
+    case MTHIP_ACT_GELU_TANH:
+      hipLaunchKernelGGL((linear_rows_kernel<MF, COLS, V, T, XT, MAXW, MTHIP_ACT_GELU_TANH>), grid, block, 0, s, a);
+      break;
+    case MTHIP_ACT_SILU:
+      hipLaunchKernelGGL((linear_rows_kernel<MF, COLS, V, T, XT, MAXW, MTHIP_ACT_SILU>), grid, block, 0, s, a);
+      break;
+    default:
+      hipLaunchKernelGGL((linear_rows_kernel<MF, COLS, V, T, XT, MAXW, MTHIP_ACT_NONE>), grid, block, 0, s, a);
   }
-}
-
-template <int V>
-int launch_rows(const GemmArgs& a, int cus, hipStream_t s) {
-  if (a.M <= 2) return launch_act<2, V>(a, cus, s);
-  if (a.M <= 4) return launch_act<4, V>(a, cus, s);
-  if (a.M <= 8) return launch_act<8, V>(a, cus, s);
-  return launch_act<16, V>(a, cus, s);
+  return check_launch("linear_rows_kernel");
 }
 
 }  // namespace
 
-// fp16, at most 16 rows, K even with rows and bases at 4-byte alignment (16-byte chunks where
-// everything is 16-byte aligned).  MTHIP_GEMM_SKINNY=0 turns it off.  Returns -1 where it does not
-// apply.
-int try_skinny_linear(int device, const GemmArgs& a, hipStream_t s) {
-  // (operands above 2 GiB are the general path's to refuse)
-  if (a.M > 16 || a.K < 2 || ((a.M - 1) * a.lda + a.K) * 2 >= (int64_t(1) << 31) ||
-      ((a.N - 1) * a.ldb + a.K) * 2 >= (int64_t(1) << 31))
-    return -1;
+// Halves per load with which the kernel takes this problem, or 0: fp16, at most 16 rows, rows and
+// bases at 16-byte alignment (8) or at 4-byte alignment (2).  The size rule is where it wins at every
+// row count against the tile GEMM with its reduction launch, weights from memory, us at M = 2 and 16
+// (SiLU, then without an activation): 320x1280 9.0 -> 4.7, 9.2 -> 5.3, 5.1 -> 4.2, 5.3 -> 4.4;
+// 1280x1280 10.5 -> 5.4, 10.8 -> 6.5, 8.0 -> 4.7, 8.3 -> 5.5; 2048x2048 (K x N) 10.9 -> 7.2,
+// 11.1 -> 8.5, 8.9 -> 7.0, 9.2 -> 8.3; 64x64 6.7 -> 3.5, 7.2 -> 4.1, 3.5 -> 3.4, 3.6 -> 3.6.  Past it
+// 16-byte loads of eight rows a wave fall behind the GEMM's tile loads: 128x8192 4.8 against 5.4
+// here, 320x6400 5.5 against 5.9, 2560x1600 9.1 against 9.3 (M = 16), 4096x4096 12.1 against 18.2.
+// MTHIP_GEMM_SKINNY=0 turns it off.
+int linear_rows_vec(const GemmArgs& a) {
+  if (a.M > 16 || a.K < 1 || a.K > 2048 || a.N > 4096 || a.N * a.K > (int64_t(1) << 22)) return 0;
   if (const char* e = std::getenv("MTHIP_GEMM_SKINNY"))
-    if (e[0] == '0') return -1;
+    if (e[0] == '0') return 0;
+  // (operands above 2 GiB are the general path's to refuse)
+  if (((a.M - 1) * a.lda + a.K) * 2 >= (int64_t(1) << 31) || ((a.N - 1) * a.ldb + a.K) * 2 >= (int64_t(1) << 31)) return 0;
   auto ok = [&](int bytes) {
     const int v = bytes / 2;
     return ((uintptr_t)a.a % bytes) == 0 && ((uintptr_t)a.b % bytes) == 0 && a.lda % v == 0 && a.ldb % v == 0 && a.K % v == 0;
   };
-  if (ok(16)) return launch_rows<8>(a, gemm_cu_count(device), s);
-  if (ok(4)) return launch_rows<2>(a, gemm_cu_count(device), s);
-  return -1;
+  return ok(16) ? 8 : ok(4) ? 2 : 0;
+}
+
+// The linear over the caller's K slices (a.ksplit of a.kt_per_split tiles) with its MFMA shape; more
+// slices than the planners choose at these sizes only when a sweep forces them.
+int launch_linear_rows(const GemmArgs& a, int mf, hipStream_t s) {
+  if (mf == 16) return launch<16, 16, 8, 10, 5, 8>(a, s);
+  if (a.ksplit <= 4) return a.rows_vec == 8 ? launch<32, 8, 8, 10, 5, 4>(a, s) : launch<32, 8, 2, 4, 2, 4>(a, s);
+  return a.rows_vec == 8 ? launch<32, 8, 8, 2, 2, 16>(a, s) : launch<32, 8, 2, 2, 2, 16>(a, s);
 }
 
 }  // namespace mthip

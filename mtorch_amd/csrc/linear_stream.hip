@@ -10,6 +10,9 @@
 #include "gemm_stream.h"
 
 namespace mthip {
+
+int launch_linear_rows(const GemmArgs& a, int mf, hipStream_t s);
+
 namespace {
 
 int env_flag(const char* name, int dflt) {
@@ -73,6 +76,11 @@ int launch_stream(int device, StreamArgs sa, GemmArgs r, int64_t K, hipStream_t 
   int bt;
   int64_t ks;
   stream_plan(M, N, K, cus, bt, ks);
+  if (!NCHW && r.rows_vec) {  // few rows: the same slices and bits
+    r.ksplit = ks;
+    r.kt_per_split = K / 64 / ks;
+    return launch_linear_rows(r, 16, s);
+  }
   sa.tiles_m = (int)ceil_div(M, bt);
   sa.tiles_n = (int)ceil_div(N, 80);
   sa.ksplit = (int)ks;

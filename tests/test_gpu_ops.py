@@ -306,8 +306,8 @@ def test_linear(dt, M, N, K):
 @pytest.mark.parametrize("M,N,K,ld", [(1, 1, 2, 2), (2, 1280, 320, 320), (3, 37, 254, 254), (5, 8200, 24, 24), (8, 130, 1544, 1552),
                                       (16, 77, 514, 516), (16, 8193, 640, 640)])
 def test_linear_few_rows(M, N, K, ld, act, monkeypatch):
-    """The few-row fp16 linear (both chunk sizes, one and two columns a wave, K and N remainders,
-    strided rows) against float64 with each op's own narrowing: the fp32 sum is off by at most
+    """The few-row fp16 linear (both load widths, K and N remainders, strided rows, and sizes past its
+    rule) against float64 with each op's own narrowing: the fp32 sum is off by at most
     K 2^-24 sum|x||w|, which may move each of the (up to two) narrowings by one fp16 step."""
     rng = np.random.default_rng(M * N + K)
     x = rng.standard_normal((M, ld)).astype(np.float16)
@@ -335,6 +335,33 @@ def test_linear_few_rows(M, N, K, ld, act, monkeypatch):
     y = F.linear_residual(xd, wd, bd, mt.from_numpy(res).to("cuda")).cpu().half_bits()
     lin = F.linear(xd, wd, bd).cpu().half_bits()
     assert np.array_equal(y, orc.f2h(orc.h2f(lin) + res.astype(np.float32)))
+
+
+@pytest.mark.parametrize("act", ["none", "gelu", "gelu_tanh", "silu"])
+@pytest.mark.parametrize("M,N,K,ld", [(2, 1280, 320, 320), (2, 1280, 1280, 1280), (16, 640, 1920, 1920), (1, 77, 8, 8),
+                                      (5, 2049, 2040, 2048), (3, 37, 254, 256), (2, 1096, 274, 274), (7, 130, 638, 638),
+                                      (9, 100, 1290, 1292), (16, 4096, 1024, 1024), (2, 4097, 320, 320), (17, 64, 640, 640)])
+def test_linear_few_rows_gives_the_tile_gemm_bits(M, N, K, ld, act, monkeypatch):
+    """Few rows take another kernel, not another sum: the bits of the tile and the streamed GEMM, with
+    K slices, K tails and rows of 4-byte alignment, an infinity and a NaN among them."""
+    rng = np.random.default_rng(M * N + K)
+    x = rng.standard_normal((M, ld)).astype(np.float16)
+    w = (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float16)
+    w[N // 2, K // 3], w[N // 3, K // 2] = np.inf, np.nan
+    b, res = rng.standard_normal(N).astype(np.float16), rng.standard_normal((M, N)).astype(np.float16)
+    xd = mt.from_numpy(x).to("cuda")[:, :K]
+    wd, bd, rd = (mt.from_numpy(t).to("cuda") for t in (w, b, res))
+    code = {"none": 0, "gelu": 1, "gelu_tanh": 2, "silu": 3}[act]
+
+    def run():
+        from mtorch_amd import _ops
+
+        return [_ops.linear(xd, wd, *a).cpu().half_bits() for a in ((None, code), (bd, code), (bd, code, rd))]
+
+    got = run()
+    monkeypatch.setenv("MTHIP_GEMM_SKINNY", "0")
+    for g, ref in zip(got, run()):
+        assert np.array_equal(g, ref)
 
 
 @pytest.mark.parametrize("M,N,K,res", [(8192, 960, 320, False), (8192, 320, 320, True), (2048, 640, 2560, True),
