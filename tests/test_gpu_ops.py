@@ -509,8 +509,9 @@ def test_matmul_unaligned_depth_every_row(dt, K):
                                       (64, 200, 1829, "4"), (257, 64, 640, "2"), (33, 300, 2, "1")])
 def test_fp32_gemm_tiles_against_float64(tile, M, N, K, ks, monkeypatch):
     """The fp32 GEMM on bf16 parts, every tile shape, at tile edges, K steps cut by K, unaligned
-    rows and K slices.  Each part product is exact, what is left out is below 2^-25 of a product,
-    and the accumulator rounds six times per 16 products: error <= (6 K / 16 + 2) 2^-24 sum|a||b|.
+    rows and K slices.  Each part product is exact, what is left out is up to 2^-24 of a product
+    (two part products of 2^-25), and the accumulator rounds six times per 16 products: error <=
+    (6 K / 16 + 2) 2^-24 sum|a||b|.
     A third of the rows is scaled by 2^-115 (the third part underflows), one row by 2^90."""
     monkeypatch.setenv("MTHIP_GEMM_F32_TILE", tile)
     monkeypatch.setenv("MTHIP_GEMM_KSPLIT", ks)
@@ -547,6 +548,89 @@ def test_fp32_gemm_non_finite_and_huge_operands(tile, monkeypatch):
     assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], exact[inf])
     fin = np.isfinite(exact)
     assert np.all(np.abs(got[fin] - exact[fin]) <= 1e-5 * np.maximum(np.abs(exact[fin]), 1.0))
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2"])
+@pytest.mark.parametrize("M,N,K,ks", [(65, 129, 31, "1"), (128, 128, 64, "1"), (64, 200, 1829, "4"), (7, 300, 5, "1")])
+def test_fp32_gemm_small_times_large(tile, M, N, K, ks, monkeypatch):
+    """Operands below 2^-110, subnormal ones among them, against partners from 1 to 2^120: the products
+    are ordinary numbers (or subnormal, or zero) and hold 24 bits as any other.  The bound is
+    test_fp32_gemm_tiles_against_float64's, and half a subnormal step per product and slice."""
+    monkeypatch.setenv("MTHIP_GEMM_F32_TILE", tile)
+    monkeypatch.setenv("MTHIP_GEMM_KSPLIT", ks)
+    rng = np.random.default_rng(M * 1000 + K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    x[::2] *= np.ldexp(np.float32(1), -110 - 4 * (np.arange(len(x[::2])) % 11))[:, None]
+    w[::3] *= np.ldexp(np.float32(1), 12 * (np.arange(len(w[::3])) % 11))[:, None]
+    w[1], x[1] = 0, 0
+    x[3 % M, K // 2] = np.float32(2.0**-147)
+    for a, b in ((x, w), (w, x)):
+        exact = a.astype(np.float64) @ b.astype(np.float64).T
+        bound = (6 * K / 16 + 3) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T) + (K + 4) * 2.0**-150
+        ad, bd = mt.from_numpy(a).to("cuda"), mt.from_numpy(b).to("cuda")
+        assert np.all(np.abs(F.linear(ad, bd).cpu().numpy() - exact) <= bound)
+        bt = mt.from_numpy(np.ascontiguousarray(b.T)).to("cuda")
+        assert np.all(np.abs(mt.matmul(ad, bt).cpu().numpy() - exact) <= bound)
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2"])
+def test_fp32_gemm_outputs_do_not_see_their_neighbours(tile, monkeypatch):
+    """A row (a column) of infinities, NaNs, huge or tiny values leaves every other output's bits alone."""
+    monkeypatch.setenv("MTHIP_GEMM_F32_TILE", tile)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((130, 200)).astype(np.float32)
+    w = rng.standard_normal((150, 200)).astype(np.float32)
+    plain = F.linear(mt.from_numpy(x).to("cuda"), mt.from_numpy(w).to("cuda")).cpu().numpy()
+    rows, cols = [3, 40, 41, 100], [5, 77, 140]
+    x[3, 7], x[40, 9], x[41], x[100] = np.nan, np.inf, x[41] * np.float32(2.0**-120), x[100] * np.float32(2.0**120)
+    w[5, 1], w[77], w[140] = -np.inf, w[77] * np.float32(2.0**-125), w[140] * np.float32(2.0**100)
+    got = F.linear(mt.from_numpy(x).to("cuda"), mt.from_numpy(w).to("cuda")).cpu().numpy()
+    keep = np.ix_(np.setdiff1d(np.arange(130), rows), np.setdiff1d(np.arange(150), cols))
+    assert np.array_equal(got[keep].view(np.uint32), plain[keep].view(np.uint32))
+
+
+@pytest.mark.parametrize("M,N", [(70, 200), (300, 130)])
+def test_fp32_gemm_outer_products_are_rounded_once(M, N):
+    """K = 1: every output is the fp32 product."""
+    rng = np.random.default_rng(M)
+    x, w = rng.standard_normal((M, 1)).astype(np.float32), rng.standard_normal((N, 1)).astype(np.float32)
+    xd, wd = mt.from_numpy(x).to("cuda"), mt.from_numpy(w).to("cuda")
+    assert np.array_equal(F.linear(xd, wd).cpu().numpy(), x * w.T)
+    assert np.array_equal(mt.matmul(xd, mt.from_numpy(np.ascontiguousarray(w.T)).to("cuda")).cpu().numpy(), x * w.T)
+
+
+@pytest.mark.parametrize("ks", ["1", "4"])
+@pytest.mark.parametrize("C,H,W,O,k,s,d", [(64, 9, 11, 70, 3, 1, 1), (64, 13, 9, 40, 3, 2, 2), (20, 11, 7, 66, 3, 2, 1),
+                                           (23, 8, 9, 33, 2, 1, 2), (96, 7, 5, 130, 1, 1, 1)])
+def test_fp32_conv_at_the_ends_of_the_range(C, H, W, O, k, s, d, ks, monkeypatch):
+    """The fp32 conv where its bf16 parts give out: an image below 2^-110 against filters up to 2^60, an
+    infinity, a NaN and values next to the fp32 maximum.  Bounds as for the linears, K = C k^2."""
+    monkeypatch.setenv("MTHIP_GEMM_KSPLIT", ks)
+    rng = np.random.default_rng(C * H + O)
+    x = rng.standard_normal((4, C, H, W)).astype(np.float32)
+    w = rng.standard_normal((O, C, k, k)).astype(np.float32)
+    w[::4] *= np.float32(2.0**60)
+    w[3] *= np.float32(2.0**-20)
+    x[1] *= np.float32(2.0**-118)
+    x[2] *= np.float32(2.0**-135)
+    x[3, 1, 2, 3], x[3, 2, 0, 1], x[3, 0, H - 1, W - 1] = np.inf, np.nan, np.float32(3.4028235e38)
+    p = d * (k - 1) // 2
+    OH, OW = (H + 2 * p - d * (k - 1) - 1) // s + 1, (W + 2 * p - d * (k - 1) - 1) // s + 1
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (p, p), (p, p)))
+    cols = np.stack([xp[:, :, y * d:y * d + (OH - 1) * s + 1:s, z * d:z * d + (OW - 1) * s + 1:s] for y in range(k) for z in range(k)], 2)
+    cols = cols.reshape(4, C * k * k, OH * OW)
+    wf = w.astype(np.float64).reshape(O, C * k * k)
+    with np.errstate(all="ignore"):
+        exact = np.stack([wf @ c for c in cols])
+        bound = (6 * C * k * k / 16 + 4) * 2.0**-24 * np.stack([np.abs(wf) @ np.abs(c) for c in cols]) + C * k * k * 2.0**-149
+        exact = np.where(np.isfinite(exact) & (np.abs(exact) > 3.4028235e38), np.sign(exact) * np.inf, exact)
+    got = F.conv2d(mt.from_numpy(x).to("cuda"), mt.from_numpy(w).to("cuda"), None, stride=s, padding=p, dilation=d)
+    got = got.cpu().numpy().astype(np.float64).reshape(exact.shape)
+    assert np.array_equal(np.isnan(got), np.isnan(exact))
+    inf, fin = np.isinf(exact), np.isfinite(exact)
+    assert np.array_equal(got[inf], exact[inf])
+    assert np.all(np.abs(got[fin] - exact[fin]) <= bound[fin])
 
 
 @pytest.mark.parametrize("dt", ["float32", "float16"])
