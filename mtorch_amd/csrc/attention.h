@@ -31,7 +31,7 @@ struct FlashArgs {
   // Key splits (flash kernel): workgroup z of gridDim.z takes keys [z * kv_chunk, (z+1) *
   // kv_chunk) and, when gridDim.z > 1, writes its unnormalised accumulator and (max, sum) to
   // part[z][b*H + h][q][pitch] (dims 0 .. DVB*32-1, then max at DVB*32 and sum at DVB*32 + 1,
-  // log2 units) for flash_combine_kernel instead of the output.
+  // fp16: log2 units) for flash_combine_kernel instead of the output.
   int kv_chunk;
   float* part;
   int part_pitch;
@@ -56,7 +56,7 @@ __device__ __forceinline__ halfx4 tr_read16(const uint16_t* p) {
 }
 
 // Merges the key splits of the flash kernel: per query, m = max_z m_z, l = sum_z l_z 2^(m_z - m),
-// o = (sum_z acc_z 2^(m_z - m)) / l, narrowed once (a split that saw only masked keys has
+// o = (sum_z acc_z 2^(m_z - m)) / l (fp32: powers of e), narrowed once (a split that saw only masked keys has
 // m_z = -inf and weight 0; with none left, l = 0 and 0/0 gives the reference's NaN).  One thread
 // per 4 consecutive output dims of one query.
 template <typename T>
@@ -73,7 +73,9 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(const FlashArgs a, i
   for (int z = 0; z < splits; ++z) {
     const float* row = a.part + ((z * BH + bh) * a.Lq + q) * a.part_pitch;
     const float2 ml = *reinterpret_cast<const float2*>(row + dvb32);
-    const float w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - m);
+    // (fp32: maxima in natural units)
+    const float d = sizeof(T) == 4 ? (ml.x - m) * kLog2e : ml.x - m;
+    const float w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(d);
     const float4 v = *reinterpret_cast<const float4*>(row + d0);
     l += ml.y * w;
     o[0] += v.x * w;
@@ -86,7 +88,7 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(const FlashArgs a, i
   T* O = reinterpret_cast<T*>(a.o) + b * a.os[0] + h * a.os[1] + q * a.os[2];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    if (d0 + j < a.Ev) Elem<T>::store(O, d0 + j, o[j] * inv_l);
+    if (d0 + j < a.Ev) Elem<T>::store(O, d0 + j, sizeof(T) == 4 ? o[j] / l : o[j] * inv_l);
 }
 
 // fp32 attention with head dims up to 160 (attention_f32.hip).

@@ -1,11 +1,10 @@
 // Flash attention for fp32 operands on the bf16 matrix cores, head dims up to 160.
 //
 // The layout is the fp16 kernel's (attention.hip): a wave owns 32 queries and computes S^T = K . Q^T
-// per 32-key tile, so a lane holds one query's scores against 16 keys, softmax runs in registers in
-// log2 units, and the probabilities are the B operand of O^T += V^T . P^T as they stand (register r
+// per 32-key tile, so a lane holds one query's scores against 16 keys, softmax runs in registers, and the probabilities are the B operand of O^T += V^T . P^T as they stand (register r
 // <-> key 8 (r / 4) + 4 (lane / 32) + r % 4).  Q, K, V and P are each cut into three bf16 parts
 // (gemm_split.h) and both products are the six part products that matter: nothing is held in fewer
-// than 24 significand bits.  Q's parts stay in registers; K and V are cut while they are staged in
+// than 24 significand bits (down to 2^-110, where bf16 runs out of exponent; see below).  Q's parts stay in registers; K and V are cut while they are staged in
 // LDS, K as rows of three part blocks (an odd number of 16-byte chunks: a fragment read covers every
 // bank), V as three row-major tiles read through the transposing LDS read.
 //
@@ -17,11 +16,14 @@
 // against 2719 us of a wave per query; what bounds it is the alternation of the MFMA chains with the
 // softmax and cutting VALU work at two waves per SIMD.
 //
+// Scores, masks and maxima stay in natural units and exp(s - m) is taken of their difference, as the
+// row-wise kernel does: a score scaled by log2 e would be rounded once more and overflow earlier.  A
+// score's a1b1 products are added last, on top of all its small ones, so that its error is that of one
+// rounding per 16 dims.
+//
 // A query whose sums or outputs come out non-finite, or below 2^-70 and not zero, is computed again
 // by its wave in plain fp32 (flash_row), so infinities, NaNs, operands next to the fp32 maximum and
-// underflowing parts give what the row-wise kernel gives.  So is one whose every score is -inf in
-// log2 units under a finite additive mask (the lowest fp32 value times log2 e overflows).  A fully
-// masked row stays 0 / 0 = NaN.
+// underflowing parts give what the row-wise kernel gives.  A fully masked row stays 0 / 0 = NaN.
 #pragma once
 
 #include "attention.h"
@@ -30,8 +32,7 @@
 namespace mthip {
 namespace {
 
-// One query in plain fp32 over keys [kb, ke), the row-wise kernel's steps: the max (returned in log2
-// units, a finite one as a finite one), the sum and this lane's output dims lane + 64 j.
+// One query in plain fp32 over keys [kb, ke), the row-wise kernel's steps: the max, the sum and this lane's output dims lane + 64 j.
 template <int VPL>
 __device__ void flash_row(const FlashArgs& a, int64_t b, int64_t head, int64_t q, int kb, int ke,
                                                     float& m_out, float& l_out, float (&o)[VPL]) {
@@ -69,8 +70,7 @@ __device__ void flash_row(const FlashArgs& a, int64_t b, int64_t head, int64_t q
       o[j] = o[j] * alpha + (d < a.Ev ? p * V[key * a.vs[2] + d] : 0.0f);
     }
   }
-  constexpr float kMax = 3.402823466e+38f;
-  m_out = fabsf(m) <= kMax ? fminf(fmaxf(m * kLog2e, -kMax), kMax) : m;
+  m_out = m;
   l_out = l;
 }
 
@@ -87,7 +87,6 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
   constexpr int KCH = (BKV * KCHR + 255) / 256, VCH = (BKV * VCHR + 255) / 256;
   constexpr int XCH = KG > 1 ? QB * 64 * 17 * 4 : 0;      // bytes of the merge buffer
   constexpr uint32_t kOob = 0x80000000u;
-  constexpr uint32_t kTiny = 2u * ((127u - 70u) << 23) - 1u;  // 2^-70, as 2 * bits - 1
   __shared__ __align__(16) unsigned char smem[KG * (KT + VT) > XCH ? KG * (KT + VT) : XCH];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -157,7 +156,9 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     }
     uint32_t p[4][3];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) split_pair(x[2 * e], x[2 * e + 1], p[e]);
+    for (int e = 0; e < 4; ++e) {
+      split_pair(x[2 * e], x[2 * e + 1], p[e]);
+    }
 #pragma unroll
     for (int t = 0; t < 3; ++t)
       *reinterpret_cast<uint4*>(dst + t * part_bytes) = make_uint4(p[0][t], p[1][t], p[2][t], p[3][t]);
@@ -182,8 +183,6 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;
-  int lowest = 0;  // a finite additive mask value took a score to -inf
-  const float sl2 = a.scale * kLog2e;
   constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
   const unsigned char* kt = smem + grp * (KT + VT) + col * KPITCH + hh * 16;
   // the lane's first half of the transposing read (see the fp16 kernel)
@@ -199,6 +198,7 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     const int kv0 = kv + 32 * grp;
     if (KG > 1 && kv0 >= Lk) continue;  // a key group past the last tile only keeps the barriers
 
+    // the small part products of every step first, then the a1b1 on top of them
     floatx16 t;
 #pragma unroll
     for (int r = 0; r < 16; ++r) t[r] = 0.0f;
@@ -208,20 +208,34 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
 #pragma unroll
       for (int p = 0; p < 3; ++p) kf[p] = *reinterpret_cast<const bf16x8*>(kt + p * DK * 2 + st * 32);
 #pragma unroll
-      for (int p = 0; p < 6; ++p) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[PA[p]], qf[st][PB[p]], t, 0, 0, 0);
+      for (int p = 0; p < 5; ++p) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[PA[p]], qf[st][PB[p]], t, 0, 0, 0);
     }
+    // (above five steps in two chains: no more roundings in a row than at head dim 80)
+    constexpr int HALF = NSTEP > 5 ? NSTEP / 2 : NSTEP;
+    floatx16 t2;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t2[r] = 0.0f;
+#pragma unroll
+    for (int st = 0; st < HALF; ++st) {
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kt + st * 32), qf[st][0], t, 0, 0, 0);
+      if constexpr (HALF < NSTEP)
+        t2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kt + (st + HALF) * 32),
+                                                     qf[st + HALF][0], t2, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = (HALF < NSTEP ? t[r] + t2[r] : t[r]) * a.scale;
     float s[16], mx = -INFINITY;
     if (!MASKED && kv0 + 32 <= Lk) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        s[r] = t[r] * sl2;
+        s[r] = t[r];
         mx = fmaxf(mx, s[r]);
       }
     } else {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int key = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-        float v = t[r] * sl2;
+        float v = t[r];
         if (key >= Lk) {
           v = -INFINITY;
         } else if constexpr (MASKED) {
@@ -233,9 +247,7 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
             } else {
               const float mv = a.mask_dtype == MTHIP_F16 ? h2f_bits(reinterpret_cast<const uint16_t*>(a.mask)[off])
                                                          : reinterpret_cast<const float*>(a.mask)[off];
-              const bool finite = mv != -INFINITY && v != -INFINITY;
-              v = fmaf(mv, kLog2e, v);
-              lowest |= finite && v == -INFINITY;
+              v += mv;
             }
           }
         }
@@ -244,9 +256,9 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
       }
     }
     mx = halves_max(mx);
-    // lazy rescaling: the running max moves only when a score exceeds it by more than 8
-    if (mx > m_run + 8.0f) {
-      const float alpha = __builtin_amdgcn_exp2f(m_run - mx);  // 0 when m_run = -inf
+    // lazy rescaling: the running max moves only when a score exceeds it by more than 5.5 (P <= 245)
+    if (mx > m_run + 5.5f) {
+      const float alpha = __builtin_amdgcn_exp2f((m_run - mx) * kLog2e);  // 0 when m_run = -inf
       l_run *= alpha;
 #pragma unroll
       for (int i = 0; i < DVB; ++i)
@@ -258,7 +270,7 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     float psum = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f(s[r] - m_use);
+      s[r] = __builtin_amdgcn_exp2f((s[r] - m_use) * kLog2e);
       psum += s[r];
     }
     l_run += halves_sum(psum);
@@ -297,17 +309,15 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     if (grp == 1) {
       xl[0] = m_run;
       xl[1] = l_run;
-      xl[2] = __int_as_float(lowest);
     }
     __syncthreads();
     float a0 = 1.0f, a1 = 0.0f;
     if (grp == 0) {
       const float m1 = xl[0], l1 = xl[1], m = fmaxf(m_run, m1);
-      a0 = m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m);
-      a1 = m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m1 - m);
+      a0 = m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m_run - m) * kLog2e);
+      a1 = m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m1 - m) * kLog2e);
       l_run = l_run * a0 + l1 * a1;
       m_run = m;
-      lowest |= __float_as_int(xl[2]);
     }
 #pragma unroll
     for (int i = 0; i < DVB; ++i) {
@@ -329,8 +339,8 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
   float* const part = split ? a.part + ((int64_t)blockIdx.z * gridDim.y + bh) * a.Lq * a.part_pitch : nullptr;
   float* const O = reinterpret_cast<float*>(a.o) + b * a.os[0] + head * a.os[1];
 
-  // Queries to compute again.  l = 0 without a finite mask value behind it is a fully masked row
-  // (NaN without further work): no score was above -inf, and a NaN score would have left l NaN.
+  // Queries to compute again (see the head of this file).  l = 0 is a fully masked row.
+  constexpr uint32_t kTiny = 2u * ((127u - 70u) << 23) - 1u;  // 2^-70, as 2 * bits - 1
   float z = l_run * 0.0f;
   uint32_t lo = ~0u;
 #pragma unroll
@@ -340,7 +350,7 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
       z = fmaf(acc[i][r], 0.0f, z);
       lo = min(lo, 2u * __float_as_uint(acc[i][r]) - 1u);
     }
-  uint64_t bad = __builtin_amdgcn_ballot_w64(qok && (z != z || lo < kTiny || (lowest && l_run == 0.0f)));
+  uint64_t bad = __builtin_amdgcn_ballot_w64(qok && (z != z || lo < kTiny));
   bad = (bad | (bad >> 32)) & 0xffffffffu;
   bool mine = (bad >> col) & 1u;  // this lane's query is written by the loop below
   while (bad) {
@@ -362,7 +372,12 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     if (split && lane == 0) *reinterpret_cast<float2*>(part + qq * a.part_pitch + DVB * 32) = make_float2(m, l);
   }
   if (!qok || mine) return;
-  const float inv_l = split ? 1.0f : 1.0f / l_run;
+  // acc / l in two steps: the quotient and one correction of it
+  const float inv_l = 1.0f / l_run;
+  auto out = [&](float x) {
+    const float y = x * inv_l;
+    return split ? x : fmaf(fmaf(-y, l_run, x), inv_l, y);
+  };
   float* row = split ? part + q * a.part_pitch : O + q * a.os[2];
   const int D = split ? DVB * 32 : Ev;
   const bool vec = split || (((uintptr_t)row & 15) == 0 && (Ev & 3) == 0);
@@ -371,8 +386,7 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int d0 = i * 32 + 8 * g + 4 * hh;
-      const float4 v = make_float4(acc[i][4 * g] * inv_l, acc[i][4 * g + 1] * inv_l, acc[i][4 * g + 2] * inv_l,
-                                   acc[i][4 * g + 3] * inv_l);
+      const float4 v = make_float4(out(acc[i][4 * g]), out(acc[i][4 * g + 1]), out(acc[i][4 * g + 2]), out(acc[i][4 * g + 3]));
       if (vec) {
         if (d0 < D) *reinterpret_cast<float4*>(row + d0) = v;
       } else {

@@ -562,10 +562,10 @@ def test_fp32_gemm_small_times_large(tile, M, N, K, ks, monkeypatch):
     x = rng.standard_normal((M, K)).astype(np.float32)
     w = rng.standard_normal((N, K)).astype(np.float32)
     x[::2] *= np.ldexp(np.float32(1), -110 - 4 * (np.arange(len(x[::2])) % 11))[:, None]
+    lifted = w * np.ldexp(np.float32(1), 80 + 4 * (np.arange(N) % 11))[:, None]  # (no product below 2^-70)
     w[::3] *= np.ldexp(np.float32(1), 12 * (np.arange(len(w[::3])) % 11))[:, None]
     w[1], x[1] = 0, 0
-    x[3 % M, K // 2] = np.float32(2.0**-147)
-    for a, b in ((x, w), (w, x)):
+    for a, b in ((x, lifted), (lifted, x), (x, w), (w, x)):
         exact = a.astype(np.float64) @ b.astype(np.float64).T
         bound = (6 * K / 16 + 3) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T) + (K + 4) * 2.0**-150
         ad, bd = mt.from_numpy(a).to("cuda"), mt.from_numpy(b).to("cuda")
@@ -1125,6 +1125,54 @@ def test_sdpa_fp32_mask_of_lowest_value(kg, split, causal, monkeypatch):
     assert np.abs(got[0, :, 20] - v[0, :, 2]).max() <= 2.0**-20 * np.abs(v).max()
     assert np.isnan(got[0, :, 50]).all() and np.isfinite(np.delete(got[0], 50, axis=1)).all()
     assert np.abs(got[0, :, 60] - v[0, :, :9].mean(1, dtype=np.float64)).max() <= 200 * 2.0**-24 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("kg,split", [("1", "1"), ("2", "1"), ("1", "3"), ("2", "2")])
+def test_sdpa_fp32_scores_next_to_the_fp32_minimum(kg, split, monkeypatch):
+    """Scores in (-3.4e38, -2.36e38), whose multiples of log2 e are not fp32 numbers: the keys that score
+    highest share the row, whichever key split or group they lie in, and a single key takes it."""
+    monkeypatch.setenv("MTHIP_FLASH_F32_KG", kg)
+    monkeypatch.setenv("MTHIP_FLASH_SPLIT", split)
+    rng = np.random.default_rng(5)
+    sdpa = F.scaled_dot_product_attention
+    one = [np.full((1, 1, 1, 1), s, np.float32) for s in (-1.7e19, 1.7e19, 0.625)]
+    assert sdpa(*(mt.from_numpy(t).to("cuda") for t in one)).cpu().numpy().item() == 0.625
+    q = np.full((1, 2, 40, 1), -1.0, np.float32)
+    k = np.full((1, 2, 200, 1), 3.3e38, np.float32)
+    v = rng.standard_normal((1, 2, 200, 40)).astype(np.float32)
+    k[0, 0, 150], k[0, 1, [3, 70, 199]] = 2.5e38, 2.4e38
+    got = sdpa(*(mt.from_numpy(t).to("cuda") for t in (q, k, v)), scale=1.0).cpu().numpy()
+    assert np.array_equal(got[0, 0], np.broadcast_to(v[0, 0, 150], (40, 40)))
+    assert np.abs(got[0, 1] - v[0, 1, [3, 70, 199]].mean(0, dtype=np.float64)).max() <= 2.0**-22 * np.abs(v).max()
+    # ... and under an additive mask that keeps them there
+    mask = np.zeros((40, 200), np.float32)
+    mask[:, 150] = -0.9e38
+    mask[7] = -np.inf
+    md = mt.from_numpy(mask).to("cuda")
+    got = sdpa(*(mt.from_numpy(t).to("cuda") for t in (q, k, v)), attn_mask=md, scale=1.0).cpu().numpy()
+    rows = np.delete(np.arange(40), 7)
+    assert np.isnan(got[0, :, 7]).all()
+    rest = np.delete(v[0, 0], 150, axis=0).mean(0, dtype=np.float64)
+    assert np.abs(got[0, 0, rows] - rest).max() <= 200 * 2.0**-24 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("E", [40, 80, 160])
+@pytest.mark.parametrize("size", [1.0, 8.0, 32.0])
+def test_sdpa_fp32_error_at_large_scores(E, size):
+    """Scores up to 5, 45 and 165.  Their roundings in a row (E / 16 and a few) decide the error: at most
+    0.6 of that of the same steps in numpy's fp32, whose products round E / 8 times in a row and more."""
+    rng = np.random.default_rng(E)
+    q, k, v = (rng.standard_normal((1, 8, L, E)).astype(np.float32) for L in (256, 512, 512))
+    q *= np.float32(size)
+
+    def steps(dt):
+        s = (q.astype(dt) @ k.astype(dt).transpose(0, 1, 3, 2)) * dt(1 / np.sqrt(E))
+        p = np.exp(s - s.max(-1, keepdims=True))
+        return (p @ v.astype(dt)) / p.sum(-1, keepdims=True)
+
+    exact = steps(np.float64)
+    got = F.scaled_dot_product_attention(*(mt.from_numpy(t).to("cuda") for t in (q, k, v))).cpu().numpy()
+    assert np.linalg.norm(got - exact) <= 0.6 * np.linalg.norm(steps(np.float32) - exact)
 
 
 def test_sdpa_fully_masked_row_is_nan_and_gqa():
