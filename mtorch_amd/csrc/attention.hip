@@ -743,9 +743,10 @@ extern "C" int mthip_sdpa(int device, int dtype, const void* q, const int64_t* q
     if (dmax <= 128) return run(std::integral_constant<int, 128>{});
     return run(std::integral_constant<int, 160>{});
   }
-  // (an infinite or NaN scale stays with the row-wise kernel here too)
+  // (a scale that is infinite, NaN or so large that it would lift what small K lose stays with the
+  // row-wise kernel)
   const bool small_heads4 = ((Lk > 0 ? Lk - 1 : 0) * std::max(ks[2], vs[2]) + dmax) * 4 < (int64_t(1) << 31);
-  if (dtype == MTHIP_F32 && Lk > 0 && dmax <= 160 && small_heads4 && ks[2] >= 0 && vs[2] >= 0 && std::isfinite(a.scale))
+  if (dtype == MTHIP_F32 && Lk > 0 && dmax <= 160 && small_heads4 && ks[2] >= 0 && vs[2] >= 0 && std::fabs(a.scale) <= 0x1p30f)
     return launch_flash_f32(device, a, bh, s);
   dim3 grid((unsigned)ceil_div(Lq, 4), (unsigned)bh);
   if (dtype == MTHIP_F16) {

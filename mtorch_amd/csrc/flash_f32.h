@@ -21,9 +21,12 @@
 // score's a1b1 products are added last, on top of all its small ones, so that its error is that of one
 // rounding per 16 dims.
 //
-// A query whose sums or outputs come out non-finite, or below 2^-70 and not zero, is computed again
-// by its wave in plain fp32 (flash_row), so infinities, NaNs, operands next to the fp32 maximum and
-// underflowing parts give what the row-wise kernel gives.  A fully masked row stays 0 / 0 = NaN.
+// A query is computed again by its wave in plain fp32 (flash_row) where the parts do not do: its sums
+// or outputs non-finite (infinities, NaNs, operands next to the fp32 maximum); Q with elements that
+// lose bits (below 2^-110) or of 2^60 and more (K may then have lost bits that matter); an output that
+// is not zero and below 2^-70 or 2^-106 of the largest |V| (bits that small probabilities lose), or zero
+// while some V lost bits.  A fully masked row stays 0 / 0 = NaN.  One NaN key thus sends every query
+// through flash_row, which is some 50 times slower.
 #pragma once
 
 #include "attention.h"
@@ -105,6 +108,8 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
 
   // Q^T fragments (B operand of S^T): query q, dims 16 st + 8 hh + [0, 8).
   bf16x8 qf[NSTEP][3];
+  uint32_t q_rest = 0;
+  float q_max = 0.0f;
 #pragma unroll
   for (int st = 0; st < NSTEP; ++st) {
     const int d0 = st * 16 + hh * 8;
@@ -113,11 +118,15 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     for (int e = 0; e < 4; ++e) {
       const float x = qok && d0 + 2 * e < E ? Q[q * a.qs[2] + d0 + 2 * e] : 0.0f;
       const float y = qok && d0 + 2 * e + 1 < E ? Q[q * a.qs[2] + d0 + 2 * e + 1] : 0.0f;
-      split_pair(x, y, p[e]);
+      split_pair(x, y, p[e], q_rest);
+      q_max = fmaxf(q_max, fmaxf(fabsf(x), fabsf(y)));
     }
 #pragma unroll
     for (int t = 0; t < 3; ++t) qf[st][t] = __builtin_bit_cast(bf16x8, make_uint4(p[0][t], p[1][t], p[2][t], p[3][t]));
   }
+
+  // (a mask of lanes at once: left to its use, the compiler holds Q's elements through the loop)
+  const uint64_t q_bad = __builtin_amdgcn_ballot_w64((q_rest & 0xffffu) != 0 || q_max >= 0x1p60f);
 
   // Staging: thread chunk c covers key c / CHR and dims 8 (c % CHR) of the step.  Loads need only
   // 4-byte alignment; a chunk that crosses E (Ev) is cleared past it.
@@ -149,7 +158,9 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
       load8(v_rsrc, c < BKV * VCHR && key < Lk, (uint32_t)(key * (int)a.vs[2] + d0), d0, Ev, vr[i]);
     }
   };
-  auto cut8 = [&](float (&x)[8], int d0, int D, unsigned char* dst, int part_bytes) {
+  uint32_t v_rest = 0;  // of the V elements this thread has cut: bits they lost, and the largest
+  float v_max = 0.0f;
+  auto cut8 = [&](auto is_v, float (&x)[8], int d0, int D, unsigned char* dst, int part_bytes) {
     if (D & 3) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = d0 + e < D ? x[e] : 0.0f;
@@ -157,7 +168,12 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     uint32_t p[4][3];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      split_pair(x[2 * e], x[2 * e + 1], p[e]);
+      if constexpr (decltype(is_v)::value) {
+        v_max = abs_max_nan(abs_max_nan(v_max, x[2 * e]), x[2 * e + 1]);
+        split_pair(x[2 * e], x[2 * e + 1], p[e], v_rest);
+      } else {
+        split_pair(x[2 * e], x[2 * e + 1], p[e]);
+      }
     }
 #pragma unroll
     for (int t = 0; t < 3; ++t)
@@ -167,13 +183,13 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
 #pragma unroll
     for (int i = 0; i < KCH; ++i) {
       const int c = tid + i * 256, key = c / KCHR, d0 = (c % KCHR) * 8;
-      if (c < BKV * KCHR) cut8(kr[i], d0, E, smem + (key >> 5) * (KT + VT) + (key & 31) * KPITCH + d0 * 2, DK * 2);
+      if (c < BKV * KCHR) cut8(std::false_type{}, kr[i], d0, E, smem + (key >> 5) * (KT + VT) + (key & 31) * KPITCH + d0 * 2, DK * 2);
     }
 #pragma unroll
     for (int i = 0; i < VCH; ++i) {
       const int c = tid + i * 256, key = c / VCHR, d0 = (c % VCHR) * 8;
       if (c < BKV * VCHR)
-        cut8(vr[i], d0, Ev, smem + (key >> 5) * (KT + VT) + KT + ((key & 31) * VRP + d0) * 2, 32 * VRP * 2);
+        cut8(std::true_type{}, vr[i], d0, Ev, smem + (key >> 5) * (KT + VT) + KT + ((key & 31) * VRP + d0) * 2, 32 * VRP * 2);
     }
   };
 
@@ -301,6 +317,20 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
     }
   }
 
+  // what the V tiles of this workgroup held
+  __shared__ float v_flags[4][2];
+  {
+    const float m = wave_reduce(v_max, [](float x, float y) { return abs_max_nan(x, y); });
+    const bool r = __builtin_amdgcn_ballot_w64((v_rest & 0xffffu) != 0) != 0;
+    if (lane == 0) {
+      v_flags[wave][0] = m;
+      v_flags[wave][1] = r ? 1.0f : 0.0f;
+    }
+    __syncthreads();
+    v_max = abs_max_nan(abs_max_nan(v_flags[0][0], v_flags[1][0]), abs_max_nan(v_flags[2][0], v_flags[3][0]));
+  }
+  const bool v_lost = v_flags[0][1] + v_flags[1][1] + v_flags[2][1] + v_flags[3][1] != 0.0f;
+
   if constexpr (KG > 1) {
     // Fold group 1's (max, sum, accumulator) into group 0: the same lane of both groups holds the
     // same query and output dims.  A group without an unmasked key has max -inf and weight 0.
@@ -340,7 +370,8 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
   float* const O = reinterpret_cast<float*>(a.o) + b * a.os[0] + head * a.os[1];
 
   // Queries to compute again (see the head of this file).  l = 0 is a fully masked row.
-  constexpr uint32_t kTiny = 2u * ((127u - 70u) << 23) - 1u;  // 2^-70, as 2 * bits - 1
+  const float low = fmaxf(0x1p-70f, 0x1p-106f * v_max);
+  const uint32_t lowb = 2u * __float_as_uint(low) - 1u;
   float z = l_run * 0.0f;
   uint32_t lo = ~0u;
 #pragma unroll
@@ -350,7 +381,14 @@ __global__ __launch_bounds__(256, DK <= 80 ? 2 : 1) void flash_fwd_f32_kernel(co
       z = fmaf(acc[i][r], 0.0f, z);
       lo = min(lo, 2u * __float_as_uint(acc[i][r]) - 1u);
     }
-  uint64_t bad = __builtin_amdgcn_ballot_w64(qok && (z != z || lo < kTiny));
+  bool again = z != z || lo < lowb;
+  if (v_lost) {
+#pragma unroll
+    for (int i = 0; i < DVB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) again |= acc[i][r] == 0.0f && i * 32 + 8 * (r >> 2) + 4 * hh + (r & 3) < Ev;
+  }
+  uint64_t bad = __builtin_amdgcn_ballot_w64(qok && again) | (q_bad & __builtin_amdgcn_ballot_w64(qok));
   bad = (bad | (bad >> 32)) & 0xffffffffu;
   bool mine = (bad >> col) & 1u;  // this lane's query is written by the loop below
   while (bad) {

@@ -1156,6 +1156,38 @@ def test_sdpa_fp32_scores_next_to_the_fp32_minimum(kg, split, monkeypatch):
     assert np.abs(got[0, 0, rows] - rest).max() <= 200 * 2.0**-24 * np.abs(v).max()
 
 
+@pytest.mark.parametrize("kg,split", [("1", "1"), ("2", "1"), ("2", "3")])
+def test_sdpa_fp32_parts_out_of_exponent(kg, split, monkeypatch):
+    """Queries below 2^-110 (subnormal ones too) on keys of 2^120, keys below 2^-110 on queries of 2^120,
+    subnormal values, and values of 2^120 under probabilities of e^-85: each as fp32 arithmetic has it.
+    Scores |s| < 12 with a few 2^-24 of sum |q||k|: outputs within 4e-6 of the largest |v| of the dim (head
+    3: the e^-85 keys carry the output, with some 6 x 85 x 2^-24 in the exponent); subnormal sums round to
+    half a step of 2^-149 twice a key, before the division by the sum of weights."""
+    monkeypatch.setenv("MTHIP_FLASH_F32_KG", kg)
+    monkeypatch.setenv("MTHIP_FLASH_SPLIT", split)
+    rng = np.random.default_rng(8)
+    q, k, v = (rng.standard_normal((1, 4, 130, 40)).astype(np.float32) for _ in range(3))
+    for h, e in ((0, -124), (1, 124)):
+        q[0, h] *= np.float32(2.0**e)
+        k[0, h] *= np.float32(2.0**-e)
+    q[0, 0, 5] *= np.float32(2.0**-8)
+    v[0, 2] *= np.float32(2.0**-136)
+    v[0, 2, :, 3] = np.float32(2.0**-140)
+    k[0, 3], q[0, 3] = 0, 0
+    q[0, 3, :, 0], k[0, 3, :, 0], k[0, 3, ::3, 0] = np.sqrt(40.0), -85.0, 0.0
+    v[0, 3] = 2.0**-20
+    v[0, 3, 1::3, :] *= np.float32(2.0**120) * (1 + rng.random((43, 40)).astype(np.float32))
+    s = q.astype(np.float64) @ k.astype(np.float64).transpose(0, 1, 3, 2) / np.sqrt(40.0)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    exact = (p / p.sum(-1, keepdims=True)) @ v.astype(np.float64)
+    got = F.scaled_dot_product_attention(*(mt.from_numpy(t).to("cuda") for t in (q, k, v))).cpu().numpy().astype(np.float64)
+    scale = np.abs(v.astype(np.float64)).max(axis=2, keepdims=True)
+    scale[0, 3] = np.abs(exact[0, 3]).max()
+    for h, tol in enumerate((4e-6, 4e-6, 4e-6, 4e-5)):
+        bound = tol * scale[0, h] + 2 * 130 * 2.0**-150 / p[0, h].sum(-1, keepdims=True) + 2.0**-149
+        assert np.all(np.abs(got[0, h] - exact[0, h]) <= bound), h
+
+
 @pytest.mark.parametrize("E", [40, 80, 160])
 @pytest.mark.parametrize("size", [1.0, 8.0, 32.0])
 def test_sdpa_fp32_error_at_large_scores(E, size):
