@@ -9,16 +9,18 @@
 #include "common.h"
 
 namespace mthip {
-// These run inside kernels built with contraction on (the GEMM epilogues): every body turns
-// it off so each multiply and add rounds separately, as the reference's x86-64 build (no FMA)
-// evaluates them.
+// These run inside kernels built with contraction on (the GEMM epilogues): every body but the fp32
+// GELU's, which names its FMAs, turns it off so each multiply and add rounds separately, as the
+// reference's x86-64 build (no FMA) evaluates them.
 
 // fp32 GELU by the reference's Linux fp32 formulas: truncated series for |x| <= 1, else
 // Abramowitz-Stegun 7.1.26 erf (tensor.cpp:17132-17154, 17265-17273).  The polynomials run in FMAs,
-// 1 / d is v_rcp with one Newton step and exp(-ax^2) a v_exp_f32 of the rounded product (off by at
-// most 6e-7 of a term below 0.37 that shrinks as that grows): under the 1.5e-7 of the erf formula
-// itself, and some 35 operations where separate rounding, an IEEE divide and expf take about 80
-// (linear + GELU 8192x1280x320 fp32: 57.1 us with the polynomials rounded at each step, 56.2 so).
+// 1 / d is v_rcp with one Newton step and exp(-ax^2) a v_exp_f32 of the rounded product, whose relative
+// error grows with ax^2 (1e-6 at ax = 2 .. 3, 4e-6 at 4 .. 6) as its share of erf, poly * e, shrinks
+// (below 5e-3, 2e-8): at most 6e-8 of erf anywhere, under the 1.5e-7 of the formula itself.  Against
+// float64 the largest error over [-20, 20] is 6.6e-7 (the truncated series at |x| = 1) either way, in
+// some 35 operations where separate rounding, an IEEE divide and expf take about 80 (linear + GELU
+// 8192x1280x320 fp32: 57.1 us with the polynomials rounded at each step, 56.2 so).
 __device__ __forceinline__ float gelu_ref_f32(float x) {
   if (fabsf(x) <= 1.0f) {
     const float inv_sqrt_two_pi = 0.39894228040143267794f;

@@ -237,6 +237,28 @@ def test_norm_upcast_pattern():
         F.layer_norm(dev(t), [320], dev(lw), dev(lb))  # the public op keeps the same-dtype rule
 
 
+@pytest.mark.parametrize("fused", [False, True])
+def test_gelu_fp32_against_float64(fused):
+    """fp32 GELU element by element, alone and in a linear's epilogue (x . 1).  Up to |x| = 1 the series'
+    first omitted term, x^14 / (sqrt(2 pi) 599040), beyond it the erf formula's 1.5e-7 (half of it times
+    |x|), and three roundings of |x| 2^-24."""
+    from scipy.special import erfc
+
+    x = np.concatenate([np.linspace(-20, 20, 400001), np.geomspace(1e-44, 3e38, 9000), -np.geomspace(1e-44, 3e38, 9000)])
+    x = np.concatenate([x.astype(np.float32), np.nextafter(np.float32([1, 1, -1, -1]), np.float32([0, 2, 0, -2])), [1, -1]])
+    x = x.astype(np.float32)
+    gelu = lambda v: (F.linear_gelu(v, one) if fused else F.gelu(v)).cpu().numpy().reshape(-1)  # noqa: E731
+    one = mt.from_numpy(np.ones((1, 1), np.float32)).to("cuda")
+    got = gelu(mt.from_numpy(x.reshape(-1, 1)).to("cuda")).astype(np.float64)
+    xd = x.astype(np.float64)
+    a = np.abs(xd)
+    exact = 0.5 * xd * erfc(-xd / np.sqrt(2.0))
+    bound = np.where(a <= 1, np.minimum(a, 1) ** 14 / (np.sqrt(2 * np.pi) * 599040), 0.75e-7 * a) + 3 * 2.0**-24 * a + 2.0**-149
+    assert np.all(np.abs(got - exact) <= bound)
+    ends = gelu(mt.from_numpy(np.array([[np.inf], [-np.inf], [np.nan], [0.0]], np.float32)).to("cuda"))
+    assert ends[0] == np.inf and np.isnan(ends[1]) and np.isnan(ends[2]) and ends[3] == 0
+
+
 def test_geglu_matches_chunk_gelu_mul():
     g = Gen(13)
     x = g.randn((2, 17, 64), "float16", 2.0)
