@@ -259,7 +259,7 @@ int launch_halo(int device, HaloArgs h, hipStream_t s) {
 
 // Unit shapes for convs of any width and channel count (BM output channels x TR x TW pixels): the
 // time of one of a unit's 9 * ceil(Cp / 64) steps and what a unit costs beside them (its first
-// loads, its epilogue), fitted to sweeps of every shape over 22 convs.
+// loads, its epilogue), fitted to sweeps of every shape over 22 convs of one or two rounds of units.
 struct HaloShape {
   int bm, tr, tw;
   double step_us, unit_us;
@@ -297,6 +297,23 @@ bool prefer_any(const HaloArgs& h, int cus) {
   return halo_time(kAnyShapes[best_any_shape(h, cus)], h, cus) < 0.85 * halo_time(own, h, cus);
 }
 
+// Whether the implicit GEMM is the faster one for a conv of any width.  Of 380 convs of 32 to 1280
+// channels and widths of 4 to 130 the halo kernel takes 0.6 of its time; it loses where few channels
+// meet many units, whose fill, patch loads and epilogues then outweigh the nine steps per block, and
+// the implicit GEMM's epilogue is its vectorised one (H W a multiple of 4).  There the modelled time
+// is short by 1.4 (1.6 where W is no multiple of 4), and the implicit GEMM runs at the rates below
+// (TFLOP/s): 4x40x72x85 -> 576 68 against 47 us, 3x48x76x97 -> 1032 139 / 78, 2x64x84x98 -> 344 38 / 26,
+// 4x72x80x106 -> 448 100 / 74; on the other side 2x112x107x104 -> 1056 130 / 151.  What it leaves is
+// at most 14 % (1x48x42x74 -> 936 19.7 / 17.2, 495 units; 4x56x53x66 -> 1176 107 / 96, H W odd).
+bool prefer_implicit(const HaloArgs& h, int cus) {
+  const HaloShape& k = kAnyShapes[best_any_shape(h, cus)];
+  const int64_t units = ceil_div(h.O, k.bm) * ceil_div(h.H, k.tr) * ceil_div(h.W, k.tw) * h.B;
+  if (h.H * h.W % 4 != 0 || units <= 2 * (int64_t)cus) return false;
+  const double tflops = h.Cp % 64 == 0 ? (h.Cp == 64 ? 330.0 : 180.0 + 2.2 * h.Cp) : h.Cp < 56 ? 225.0 : 290.0;
+  const double gemm_us = 18.0 * h.B * h.H * h.W * h.O * h.Cp / tflops / 1.0e6;
+  return halo_time(k, h, cus) * (h.W % 4 == 0 ? 1.4 : 1.6) > gemm_us;
+}
+
 template <int ANYW>
 int launch_halo_any(int device, const HaloArgs& h, hipStream_t s) {
   const char* f = std::getenv("MTHIP_CONV_HALO_SHAPE");
@@ -314,7 +331,7 @@ int launch_halo_any(int device, const HaloArgs& h, hipStream_t s) {
 // sends every conv to the implicit GEMM): the width's own instance where the padded channel count
 // is a whole number of 64-channel blocks and the width one of the SD latent widths, the any-width
 // instances otherwise, from 32 input channels (below, the zeros of the 64-channel block outweigh
-// what the implicit GEMM re-reads).
+// what the implicit GEMM re-reads) and where prefer_implicit does not say otherwise.
 int try_conv_halo(int device, const void* xp, const void* wp, const void* b, void* y, int64_t B, int64_t H, int64_t W,
                   int64_t Cp, int64_t O, int64_t KH, int64_t KW, int64_t sh, int64_t sw, int64_t ph, int64_t pw,
                   int64_t dh, int64_t dw, const void* residual, const void* chan_add, int64_t chan_add_ld,
@@ -324,8 +341,8 @@ int try_conv_halo(int device, const void* xp, const void* wp, const void* b, voi
     return e == nullptr || std::atoi(e) != 0;
   }();
   if (!enabled || KH != 3 || KW != 3 || sh != 1 || sw != 1 || ph != 1 || pw != 1 || dh != 1 || dw != 1) return -1;
-  const bool any_width = Cp % 64 != 0 || O < 64 || !(W == 64 || W == 32 || W == 16 || W == 8) ||
-                         std::getenv("MTHIP_CONV_HALO_ANY") != nullptr;
+  const bool forced = std::getenv("MTHIP_CONV_HALO_ANY") != nullptr;
+  const bool any_width = Cp % 64 != 0 || O < 64 || !(W == 64 || W == 32 || W == 16 || W == 8) || forced;
   if (any_width && (Cp < 32 || O < 32)) return -1;
   if (((uintptr_t)b & 1) || ((uintptr_t)residual & 7) || ((uintptr_t)xp & 15) || ((uintptr_t)wp & 15)) return -1;
   if (B * H * W * Cp * 2 >= (int64_t(1) << 31) || O * 9 * Cp * 2 >= (int64_t(1) << 31) ||
@@ -346,6 +363,7 @@ int try_conv_halo(int device, const void* xp, const void* wp, const void* b, voi
   h.O = (int)O;
   h.x_bytes = (int)(B * H * W * Cp * 2);
   h.w_bytes = (int)(O * 9 * Cp * 2);
+  if (any_width && !forced && prefer_implicit(h, halo_cu_count(device))) return -1;
   if (any_width || prefer_any(h, halo_cu_count(device)))
     return W % 4 == 0 ? launch_halo_any<1>(device, h, s) : launch_halo_any<2>(device, h, s);
   switch (W) {

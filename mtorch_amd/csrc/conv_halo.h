@@ -173,7 +173,7 @@ struct HaloSchedule {
 // ANYW: 0 -- the image width is TW and Cp a multiple of 64.  1 and 2 -- any width, covered by
 // col_blocks units of TW columns, and any Cp (the chunks of the last channel block past Cp are
 // fetched as zeros); 1 needs W % 4 == 0 (every group of four pixels lies in one image row, 8-byte
-// aligned), 2 stores single pixels and reads HAS_R as "the epilogue may add either operand".
+// aligned), 2 stores groups at any alignment and reads HAS_R as "the epilogue may add either operand".
 template <int BM, int TR, int TW, int WGM, int SW, bool HAS_A, bool HAS_R, int NPW, int ANYW = 0>
 __global__ __launch_bounds__(64 * (4 + NPW)) void conv3x3_halo_kernel(const HaloArgs args) {
   constexpr int NW = 4;                 // compute waves (the others are producers)
@@ -409,12 +409,18 @@ __global__ __launch_bounds__(64 * (4 + NPW)) void conv3x3_halo_kernel(const Halo
       for (int fc = 0; fc < FC; ++fc) {
         const int orr = oc[fc] < O ? oc[fc] : O - 1;
         if constexpr (ANYW == 2) {
-          uint32_t h[4];
+          // (absent: nothing adds it; the group that the image cuts pixel by pixel)
+          rz[fp][fc].u = make_uint2(0u, 0u);
+          if (!res) continue;
+          const T* src = res + ((int64_t)img * O + orr) * HW + oy * W + ox;
+          if (ox + 4 <= W) {
+            __builtin_memcpy(&rz[fp][fc].u, src, 8);
+          } else {
+            uint32_t h[4];
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
-            h[t] = __builtin_amdgcn_raw_buffer_load_b16(
-                r_rsrc, (((img * O + orr) * HW) + oy * W + min(ox + t, W - 1)) * 2, 0, 0);
-          rz[fp][fc].u = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+            for (int t = 0; t < 4; ++t) h[t] = src[min(t, W - 1 - ox)];
+            rz[fp][fc].u = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+          }
           continue;
         }
         const auto u = __builtin_amdgcn_raw_buffer_load_b64(r_rsrc, (((img * O + orr) * HW) + oy * W + ox) * 2, 0, 0);
@@ -533,9 +539,12 @@ __global__ __launch_bounds__(64 * (4 + NPW)) void conv3x3_halo_kernel(const Halo
         const int oy = y0 + qq / TW, ox = x0 + qq % TW;
         if (oy < H && (!ANYW || ox < W)) {
           float* dst = args.partial + ((int64_t)split * O + o) * args.ld_partial + (int64_t)img * HW + oy * W + ox;
-          if constexpr (ANYW == 2) {
+          if (ANYW == 2 && ox + 4 <= W) {
+            const float4 v = make_float4(acc[fp][fc][0], acc[fp][fc][1], acc[fp][fc][2], acc[fp][fc][3]);
+            __builtin_memcpy(dst, &v, 16);
+          } else if (ANYW == 2) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 3; ++t)
               if (ox + t < W) dst[t] = acc[fp][fc][t];
           } else {
             *reinterpret_cast<float4*>(dst) = make_float4(acc[fp][fc][0], acc[fp][fc][1], acc[fp][fc][2], acc[fp][fc][3]);
@@ -623,7 +632,8 @@ __global__ __launch_bounds__(64 * (4 + NPW)) void conv3x3_halo_kernel(const Halo
   // y0*W + q.  When Y is 8-byte aligned each is one 8-byte buffer store whose address is one
   // per-lane offset (+ fp*32 bytes, + fc*16 channels in soffset); rows past H and channels past
   // O get an out-of-range offset, which the store drops.
-  // ANYW == 1: the same with the pixel's own offset; ANYW == 2: pixel by pixel.
+  // ANYW == 1: the same with the pixel's own offset; ANYW == 2 (and any Y): two-byte aligned
+  // groups, those the image cuts pixel by pixel.
   if (ANYW != 2 && ((uintptr_t)Y & 7) == 0) {
     const __amdgpu_buffer_rsrc_t y_rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)Y, (short)0, args.B * O * HW * 2, 0x00020000);
@@ -650,11 +660,14 @@ __global__ __launch_bounds__(64 * (4 + NPW)) void conv3x3_halo_kernel(const Halo
     for (int fc = 0; fc < FC; ++fc) {
       if (oy < H && oc[fc] < O) {
         T* dst = Y + ((int64_t)img * O + oc[fc]) * HW + oy * W + ox;
-        const T v[4] = {(T)(out[fp][fc].x & 0xffffu), (T)(out[fp][fc].x >> 16), (T)(out[fp][fc].y & 0xffffu),
-                        (T)(out[fp][fc].y >> 16)};
+        if (!ANYW || ox + 4 <= W) {
+          __builtin_memcpy(dst, &out[fp][fc], 8);  // (two-byte alignment will do)
+        } else {
+          const T v[3] = {(T)(out[fp][fc].x & 0xffffu), (T)(out[fp][fc].x >> 16), (T)(out[fp][fc].y & 0xffffu)};
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          if (!ANYW || ox + t < W) dst[t] = v[t];
+          for (int t = 0; t < 3; ++t)
+            if (ox + t < W) dst[t] = v[t];
+        }
       }
     }
   }

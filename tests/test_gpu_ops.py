@@ -1466,16 +1466,49 @@ def test_conv3x3_halo_kernel_shapes(B, C, H, W, O):
     assert rel(val(fused), ref) <= 1e-2
 
 
+def run_conv3x3_nhwc(x, w, b, ca, res, dirty=7.0):
+    """The channels-last 3x3 conv entry on fp16 arrays; ca and res may be None."""
+    from mtorch_amd import _lib
+
+    (B, C, H, W), O = x.shape, w.shape[0]
+    L, cp = _lib.lib(), -(-C // 8) * 8
+    xn = np.zeros((B, H, W, cp), np.float16)
+    xn[..., :C] = x.transpose(0, 2, 3, 1)
+    dev = lambda t: None if t is None else mt.from_numpy(np.ascontiguousarray(t).view(np.uint16), dtype=mt.float16).to("cuda")  # noqa: E731
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    xd, wd, bd, cd, rd = dev(xn), dev(w), dev(b), dev(ca), dev(res)
+    wp = mt.empty(O * 9 * cp, dtype=mt.float16, device="cuda")
+    y = mt.full([B, O, H, W], dirty, dtype=mt.float16).to("cuda")
+    _lib.check(L.mthip_conv2d_pack_weight(0, 0, wd.data_ptr(), wp.data_ptr(), O, C, 3, 3))
+    _lib.check(L.mthip_conv2d_nhwc(0, 0, xd.data_ptr(), wp.data_ptr(), bd.data_ptr(), y.data_ptr(), B, C, H, W, O, 3, 3, 1, 1,
+                                   1, 1, 1, 1, ptr(rd), ptr(cd), O))
+    return y.cpu().half_bits().view(np.float16)
+
+
+def conv3x3_float64(x, w):
+    (B, C, H, W), O = x.shape, w.shape[0]
+    xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    y = np.zeros((B, O, H * W))
+    for ky in range(3):
+        for kx in range(3):
+            y += w[:, :, ky, kx].astype(np.float64) @ xp[:, :, ky:ky + H, kx:kx + W].reshape(B, C, H * W)
+    return y.reshape(B, O, H, W)
+
+
 @pytest.mark.parametrize("shape", range(6))
-@pytest.mark.parametrize("B,C,H,W,O", [(1, 32, 5, 7, 48), (2, 72, 9, 36, 100), (1, 200, 17, 33, 64), (2, 64, 8, 12, 80),
-                                       (1, 96, 3, 98, 81), (1, 136, 6, 5, 70)])
-def test_conv3x3_halo_any_width(shape, B, C, H, W, O, monkeypatch):
+@pytest.mark.parametrize("B,C,H,W,O,ks", [(1, 32, 5, 7, 48, None), (2, 72, 9, 36, 100, None), (1, 200, 17, 33, 64, None),
+                                          (2, 64, 8, 12, 80, None), (1, 96, 3, 98, 81, None), (1, 136, 6, 5, 70, None),
+                                          (2, 136, 7, 21, 90, "1"), (1, 200, 9, 40, 64, "1"), (2, 264, 5, 18, 50, "1"),
+                                          (3, 264, 6, 9, 33, "2"), (1, 384, 4, 44, 48, "1")])
+def test_conv3x3_halo_any_width(shape, B, C, H, W, O, ks, monkeypatch):
     """The any-width halo instances: column blocks cut by the image, channel blocks cut by Cp, odd
-    widths (single-pixel stores), K splits, with bias, channel add and residual -- bit for bit the
-    rounding chain of the separate ops on one-hot weights (each output one exact product), and
-    against float64 on random ones."""
+    widths over several images, K splits and units that walk two to six channel blocks, with and without
+    channel add and residual -- bit for bit the rounding chain of the separate ops on one-hot weights
+    (each output one exact product), and against float64 on random ones."""
     monkeypatch.setenv("MTHIP_CONV_HALO_ANY", "1")
     monkeypatch.setenv("MTHIP_CONV_HALO_SHAPE", str(shape))
+    if ks:
+        monkeypatch.setenv("MTHIP_CONV_HALO_KSPLIT", ks)
     rng = np.random.default_rng(B * C + W)
     x = rng.standard_normal((B, C, H, W)).astype(np.float16)
     b = rng.standard_normal(O).astype(np.float16)
@@ -1486,39 +1519,39 @@ def test_conv3x3_halo_any_width(shape, B, C, H, W, O, monkeypatch):
     for o in range(O):
         one[o, (7 * o) % C, o % 3, (o // 3) % 3] = rng.standard_normal()
 
-    def run(wt):
-        from mtorch_amd import _lib
-
-        L, cp = _lib.lib(), -(-C // 8) * 8
-        xn = np.zeros((B, H, W, cp), np.float16)
-        xn[..., :C] = x.transpose(0, 2, 3, 1)
-        d = [mt.from_numpy(np.ascontiguousarray(t).view(np.uint16), dtype=mt.float16).to("cuda") for t in (xn, wt, b, ca, res)]
-        wp = mt.empty(O * 9 * cp, dtype=mt.float16, device="cuda")
-        y = mt.full([B, O, H, W], 7.0, dtype=mt.float16).to("cuda")
-        _lib.check(L.mthip_conv2d_pack_weight(0, 0, d[1].data_ptr(), wp.data_ptr(), O, C, 3, 3))
-        _lib.check(L.mthip_conv2d_nhwc(0, 0, d[0].data_ptr(), wp.data_ptr(), d[2].data_ptr(), y.data_ptr(), B, C, H, W, O,
-                                       3, 3, 1, 1, 1, 1, 1, 1, d[4].data_ptr(), d[3].data_ptr(), O))
-        return y.cpu().half_bits().view(np.float16)
-
-    def conv(wt):
-        xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 1), (1, 1)))
-        y = np.zeros((B, O, H, W))
-        for ky in range(3):
-            for kx in range(3):
-                y += np.einsum("oc,bchw->bohw", wt[:, :, ky, kx].astype(np.float64), xp[:, :, ky:ky + H, kx:kx + W])
-        return y
-
     def narrow(v):
         return orc.h2f(orc.f2h(v.astype(np.float32))).astype(np.float32)
 
-    # one product per output, exact in fp32; each add in fp32, narrowed as the separate ops narrow
-    v = conv(one).astype(np.float32) + b.astype(np.float32).reshape(1, -1, 1, 1)
-    v = narrow(v) + ca.astype(np.float32)[:, :, None, None]
-    v = narrow(v) + res.astype(np.float32)
-    assert np.array_equal(run(one), orc.f2h(v.astype(np.float32)).view(np.float16))
-    exact = conv(w) + b.astype(np.float64).reshape(1, -1, 1, 1) + ca.astype(np.float64)[:, :, None, None] + res.astype(np.float64)
-    # three narrowings of half an ulp each at |value| < 16 and the fp32 sum
-    assert np.all(np.abs(run(w).astype(np.float64) - exact) <= 3 * 2.0**-11 * np.maximum(np.abs(exact), 4.0))
+    product, exact = conv3x3_float64(x, one).astype(np.float32), conv3x3_float64(x, w)
+    for c, r in ((ca, res), (None, res), (ca, None), (None, None)):
+        # one product per output, exact in fp32; each add in fp32, narrowed as the separate ops narrow
+        v = product + b.astype(np.float32).reshape(1, -1, 1, 1)
+        e = exact + b.astype(np.float64).reshape(1, -1, 1, 1)
+        if c is not None:
+            v = narrow(v) + c.astype(np.float32)[:, :, None, None]
+            e = e + c.astype(np.float64)[:, :, None, None]
+        if r is not None:
+            v = narrow(v) + r.astype(np.float32)
+            e = e + r.astype(np.float64)
+        assert np.array_equal(run_conv3x3_nhwc(x, one, b, c, r), orc.f2h(v.astype(np.float32)).view(np.float16))
+        # three narrowings of half an ulp each at |value| < 16 and the fp32 sum
+        got = run_conv3x3_nhwc(x, w, b, c, r).astype(np.float64)
+        assert np.all(np.abs(got - e) <= 3 * 2.0**-11 * np.maximum(np.abs(e), 4.0))
+
+
+@pytest.mark.parametrize("B,C,H,W,O", [(2, 640, 48, 32, 640), (2, 64, 70, 64, 256), (1, 40, 72, 85, 700), (1, 64, 84, 98, 700)])
+def test_conv3x3_rules_between_kernels(B, C, H, W, O):
+    """Sizes where latent widths leave their own instance for an any-width shape, and where few channels
+    under many units stay with the implicit GEMM: some output channels against float64."""
+    rng = np.random.default_rng(C + W)
+    x = rng.standard_normal((B, C, H, W)).astype(np.float16)
+    b = rng.standard_normal(O).astype(np.float16)
+    res = rng.standard_normal((B, O, H, W)).astype(np.float16)
+    w = (rng.standard_normal((O, C, 3, 3)) / np.sqrt(9 * C)).astype(np.float16)
+    some = np.unique(np.concatenate([np.arange(0, O, 37), [O - 1]]))
+    exact = conv3x3_float64(x, w[some]) + b[some].astype(np.float64).reshape(1, -1, 1, 1) + res[:, some].astype(np.float64)
+    got = run_conv3x3_nhwc(x, w, b, None, res)[:, some].astype(np.float64)
+    assert np.all(np.abs(got - exact) <= 2 * 2.0**-11 * np.maximum(np.abs(exact), 4.0))
 
 
 @pytest.mark.parametrize("C,H", [(640, 16), (1280, 16), (1280, 13)])
