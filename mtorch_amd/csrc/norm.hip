@@ -275,10 +275,11 @@ __global__ __launch_bounds__(256) void group_norm_apply_kernel(const T* __restri
 // |SiLU(x)| <= |x|) -- is found by a running maximum of |value| and a packed minimum of the halves'
 // difference bits to 0xc173: a wave in which some lane met one redoes the unit with f2h_fast and
 // silu_half.  Equal to them for every other input (tests/f2h_fast_model.c; test_gpu_ops.py's
-// exhaustive SiLU cases).  The arithmetic bounds the large-batch GroupNorm + SiLU: with f2h_fast and
+// exhaustive SiLU cases); `again` fills outs anew for that, so that they need not be held beside the
+// narrowed values.  The arithmetic bounds the large-batch GroupNorm + SiLU: with f2h_fast and
 // silu_half on every value 60 us at 32x320x64x64, so evaluated 53 (32 us of HBM traffic).
-template <int U, bool SILU>
-__device__ __forceinline__ void gn_narrow(const float (&outs)[U], uint32_t (&hv)[U]) {
+template <int U, bool SILU, typename F>
+__device__ __forceinline__ void gn_narrow(float (&outs)[U], uint32_t (&hv)[U], F again) {
   typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
   float amax = 0.0f;
   u16x2 pinned = {0xffffu, 0xffffu};
@@ -305,6 +306,7 @@ __device__ __forceinline__ void gn_narrow(const float (&outs)[U], uint32_t (&hv)
   }
   const bool rare = SILU ? !(amax < 60.0f) || pinned[0] == 0 || pinned[1] == 0 : !(amax < 65520.0f);
   if (__builtin_amdgcn_ballot_w64(rare)) {
+    again(outs);
 #pragma unroll
     for (int j = 0; j < U; ++j) {
       uint16_t o = f2h_fast(outs[j]);
@@ -336,7 +338,9 @@ void group_norm_single_kernel(const T* __restrict__ x, const P* __restrict__ gam
   __shared__ float red_s[NPART * CPT][4], red_ss[NPART * CPT][4];
   __shared__ float2 st_s;
   const int64_t bg = blockIdx.x;
-  const int t = threadIdx.x & 255, part = threadIdx.x >> 8, wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
+  // (the part is the wave's: its chunk bounds live in scalar registers)
+  const int t = threadIdx.x & 255, part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+  const int wave = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
   const T* xb = x + bg * group_size;
   T* yb = y + bg * group_size;
   uint4 d[CPT][IPC];
@@ -350,7 +354,7 @@ void group_norm_single_kernel(const T* __restrict__ x, const P* __restrict__ gam
       const int i = begin + (t + it * 256) * V;
       d[kk][it] = make_uint4(0u, 0u, 0u, 0u);
       if (k < splits && i < end) {
-        d[kk][it] = *reinterpret_cast<const uint4*>(xb + i);
+        d[kk][it] = *reinterpret_cast<const uint4*>(xb + (uint32_t)i);
       }
     }
   }
@@ -410,27 +414,37 @@ void group_norm_single_kernel(const T* __restrict__ x, const P* __restrict__ gam
   // vectors must stay in registers)
   auto apply = [&](auto silu_c) {
     constexpr bool SILU = decltype(silu_c)::value;
+    int at = t;
+    asm volatile("" : "+v"(at));  // (the loads' offsets are computed again, not held beside the vectors)
 #pragma unroll
     for (int kk = 0; kk < CPT; ++kk) {
       const int k = NPART * kk + part;
       const int begin = k * (int)chunk, end = min(begin + (int)chunk, (int)group_size);  // (<= 20 chunks of <= 2048)
 #pragma unroll
       for (int it = 0; it < IPC; ++it) {
-        const int i = begin + (t + it * 256) * V;
+        const int i = begin + (at + it * 256) * V;
         if (k < splits && i < end) {
-          const int c = c0 + (int)div_inner.div((uint32_t)i);
+          const uint32_t c = (uint32_t)c0 + div_inner.div((uint32_t)i);
           const float gm = gamma ? Elem<P>::load(gamma, c) : 1.0f;
           const float bt = beta ? Elem<P>::load(beta, c) : 0.0f;
           float f[V];
-          Vec16<T>::unpack(d[kk][it], f);
           if constexpr (sizeof(T) == 2) {
             uint32_t h[V];
+            auto values = [&](float (&o)[V], uint4 v) {
+              Vec16<T>::unpack(v, o);
 #pragma unroll
-            for (int j = 0; j < V; ++j) f[j] = gn_value<T, P>(f[j], mean, inv, gm, bt, 0);
-            gn_narrow<V, SILU>(f, h);
-            *reinterpret_cast<uint4*>(yb + i) =
+              for (int j = 0; j < V; ++j) o[j] = gn_value<T, P>(o[j], mean, inv, gm, bt, 0);
+            };
+            values(f, d[kk][it]);
+            gn_narrow<V, SILU>(f, h, [&](float (&o)[V]) {
+              uint4 v = d[kk][it];
+              asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));  // (computed here, not carried)
+              values(o, v);
+            });
+            *reinterpret_cast<uint4*>(yb + (uint32_t)i) =
                 make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
           } else {
+            Vec16<T>::unpack(d[kk][it], f);
 #pragma unroll
             for (int j = 0; j < V; ++j) f[j] = gn_value<T, P>(f[j], mean, inv, gm, bt, SILU ? 1 : 0);
             Vec16<T>::store(yb + i, f);
@@ -1209,7 +1223,7 @@ __global__ __launch_bounds__(1024) void group_norm_nhwc_onepass_kernel(
         else
           outs[j] = (v - mean) * inv * cs.x + cs.y;
       }
-      gn_narrow<U, SILU>(outs, hv);
+      gn_narrow<U, SILU>(outs, hv, [](float (&)[U]) {});
       const int64_t off = ((int64_t)b * HW + p_lo + pl) * Cp + g * gc + u * U;
       if constexpr (U == 2) {
         *reinterpret_cast<uint32_t*>(y + off) = hv[0] | (hv[1] << 16);
