@@ -264,7 +264,10 @@ int mthip_gemm(int device, int dtype, int64_t batch, int64_t M, int64_t N, int64
     // zeros there; unpadded rows have K a multiple of the chunk).
     // (fp32 rows end at K, and N: their last chunk may be cut by the range check.)
     a.a_bytes = ((M - 1) * a.lda + (f32 ? K : ceil_div(a.K, vec) * vec)) * es;
-    a.b_bytes = b_trans ? ((N - 1) * a.ldb + a.K) * es : ((K - 1) * a.ldb + (f32 ? N : ceil_div(N, vec) * vec)) * es;
+    // (K = 0: B has no rows, and an extent of less than nothing would let every read pass the check)
+    a.b_bytes = b_trans  ? ((N - 1) * a.ldb + a.K) * es
+                : K == 0 ? 0
+                         : ((K - 1) * a.ldb + (f32 ? N : ceil_div(N, vec) * vec)) * es;
     if (a.a_bytes > kMaxBufferBytes || a.b_bytes > kMaxBufferBytes) {
       rc = fail(MTHIP_ERR_UNSUPPORTED, "mthip_gemm: operands above 2 GiB per batch are not supported");
     } else {

@@ -656,6 +656,25 @@ def test_fp32_conv_at_the_ends_of_the_range(C, H, W, O, k, s, d, ks, monkeypatch
 
 
 @pytest.mark.parametrize("dt", ["float32", "float16"])
+@pytest.mark.parametrize("beta", [0.0, 2.0])
+def test_gemm_without_depth(dt, beta):
+    """K = 0 with a row stride beyond the row: beta * c_in (zeros without it), nothing read of a and b."""
+    from mtorch_amd import _lib
+
+    M, N, ldb = 70, 40, 48
+    c = np.random.default_rng(2).standard_normal((M, N)).astype(np.float16 if dt == "float16" else np.float32)
+    cd = mt.from_numpy(c).to("cuda")
+    ab = mt.full([64], 3.0, dtype=getattr(mt, dt)).to("cuda")
+    y = mt.full([M, N], 7.0, dtype=getattr(mt, dt)).to("cuda")
+    cin = (cd.data_ptr(), N, 1, 0) if beta else (None, 0, 0, 0)
+    code = {"float16": _lib.F16, "float32": _lib.F32}[dt]
+    _lib.check(_lib.lib().mthip_gemm(0, code, 1, M, N, 0, ab.data_ptr(), 8, 0, ab.data_ptr(), ldb, 0, 0, y.data_ptr(), N, 0,
+                                     1.0, beta, *cin))
+    got = y.cpu().half_bits().view(np.float16) if dt == "float16" else y.cpu().numpy()
+    assert np.array_equal(got, (beta * c).astype(c.dtype))
+
+
+@pytest.mark.parametrize("dt", ["float32", "float16"])
 def test_addmm_and_baddbmm(dt):
     g = Gen(32)
     inp = g.randn((40,), dt)
