@@ -12,8 +12,8 @@
 // and two key tiles, each pair of waves with its own running softmax, merged through LDS at the end
 // -- for grids that would leave SIMDs without a wave.
 //
-// 2x8 heads, 1024x1024, head dim 80: 57 us (5.4 GFLOP as 32 GFLOP of bf16 products, 570 TFLOP/s)
-// against 2719 us of a wave per query; what bounds it is the alternation of the MFMA chains with the
+// 2x8 heads, 1024x1024, head dim 80: 56 us (5.4 GFLOP as 32 GFLOP of bf16 products, 580 TFLOP/s)
+// against 2709 us of a wave per query; what bounds it is the alternation of the MFMA chains with the
 // softmax and cutting VALU work at two waves per SIMD.
 //
 // Scores, masks and maxima stay in natural units and exp(s - m) is taken of their difference, as the

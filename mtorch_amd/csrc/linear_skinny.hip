@@ -148,12 +148,12 @@ int launch(const GemmArgs& a, hipStream_t s) {
 
 // Halves per load with which the kernel takes this problem, or 0: fp16, at most 16 rows, rows and
 // bases at 16-byte alignment (8) or at 4-byte alignment (2).  The size rule is where it wins at every
-// row count against the tile GEMM with its reduction launch, weights from memory, us at M = 2 and 16
-// (SiLU, then without an activation): 320x1280 9.0 -> 4.7, 9.2 -> 5.3, 5.1 -> 4.2, 5.3 -> 4.4;
-// 1280x1280 10.5 -> 5.4, 10.8 -> 6.5, 8.0 -> 4.7, 8.3 -> 5.5; 2048x2048 (K x N) 10.9 -> 7.2,
-// 11.1 -> 8.5, 8.9 -> 7.0, 9.2 -> 8.3; 64x64 6.7 -> 3.5, 7.2 -> 4.1, 3.5 -> 3.4, 3.6 -> 3.6.  Past it
-// 16-byte loads of eight rows a wave fall behind the GEMM's tile loads: 128x8192 4.8 against 5.4
-// here, 320x6400 5.5 against 5.9, 2560x1600 9.1 against 9.3 (M = 16), 4096x4096 12.1 against 18.2.
+// row count against the GEMM with its reduction launch, weights from memory, us at M = 2 and 16 (SiLU,
+// then without an activation): 320x1280 9.1 -> 4.5, 9.4 -> 4.9, 5.4 -> 4.2, 5.5 -> 4.5; 1280x1280
+// 10.6 -> 5.4, 10.9 -> 6.1, 8.0 -> 4.7, 8.4 -> 5.5; 2048x2048 10.8 -> 7.4, 11.2 -> 8.5, 8.9 -> 7.0,
+// 9.2 -> 8.1; 64x64 6.8 -> 3.7, 7.3 -> 4.2, 3.5 -> 3.4, 3.7 -> 3.6.  Past it (K x N) 16-byte loads of
+// eight rows a wave fall behind the GEMM's tile loads: 128x8192 4.8 against 5.4 here, 320x6400 5.5
+// against 5.9, 2560x1600 9.1 against 9.3 (M = 16), 4096x4096 12.1 against 18.2.
 // MTHIP_GEMM_SKINNY=0 turns it off.
 int linear_rows_vec(const GemmArgs& a) {
   if (a.M > 16 || a.K < 1 || a.K > 2048 || a.N > 4096 || a.N * a.K > (int64_t(1) << 22)) return 0;
